@@ -68,7 +68,7 @@ struct dg_handle {
   double *d_k[4] = {nullptr, nullptr, nullptr, nullptr};
   double *d_err = nullptr, *d_lam = nullptr;
   double *d_prev = nullptr;  // step base copy (convergence norm on the limiter path)
-  DevState *d_st = nullptr;
+  DevState *d_st = nullptr;  // [2]: the state between steps, the running step's (k_stage_s)
   unsigned long long *d_part = nullptr;  // per-block maxima of the step reduction
   int *d_bad = nullptr;                  // positivity flags of the stored state d_c
   // graphs of 2^q steps, q < kGraphLevels (same configuration key)
@@ -329,7 +329,7 @@ extern "C" int dg_create(dg_handle **out, const dg_config *cfg) {
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreate(&h->ev0) != hipSuccess || hipEventCreate(&h->ev1) != hipSuccess ||
       ensure_tables(cfg->device, cfg->p) != 0 || ensure_scratch(cfg->device) != 0 ||
-      hipMalloc((void **)&h->d_st, sizeof(DevState)) != hipSuccess) {
+      hipMalloc((void **)&h->d_st, 2 * sizeof(DevState)) != hipSuccess) {
     dg_destroy(h);
     return DG_ERR_HIP;
   }
@@ -574,8 +574,10 @@ extern "C" int dg_set_mesh(dg_handle *h, int K, const double *V, const int *es, 
   if ((rc = alloc(h, (void **)&h->d_err, sizeof(double) * (size_t)K * h->N)) != DG_OK) return rc;
   if ((rc = alloc(h, (void **)&h->d_lam, kd)) != DG_OK) return rc;
   if ((rc = alloc(h, (void **)&h->d_bad, sizeof(int) * (size_t)K)) != DG_OK) return rc;
-  if ((rc = alloc(h, (void **)&h->d_part,
-                  sizeof(unsigned long long) * 2 * (size_t)((K + 63) / 64))) != DG_OK)
+  const size_t nparts = K <= small_max_k(h->cfg.physics, h->cfg.p)
+                            ? std::max(small_blocks(h->cfg.p, K), (K + 63) / 64)
+                            : (K + 63) / 64;
+  if ((rc = alloc(h, (void **)&h->d_part, sizeof(unsigned long long) * 2 * nparts)) != DG_OK)
     return rc;
   HIPCHK(h, hipMemset(h->d_c, 0, sb));
   // every buffer is in place: the handle has a mesh from here on
@@ -685,6 +687,18 @@ extern "C" int dg_get_coeffs(dg_handle *h, double *C, int where) {
 // (dg_config.volume; the library's choice is the vector FMAs)
 static bool volume_mfma(const dg_config &c) { return c.volume == 2; }
 
+// Whether the handle's stages run the point-parallel kernel: small meshes,
+// unless the caller asked for the matrix cores or (DG_STAGE_GATHER) for the
+// four-lane kernel's gather form.
+static bool small_path(const dg_handle *h) {
+  if (h->K > small_max_k(h->cfg.physics, h->cfg.p) || volume_mfma(h->cfg)) return false;
+  return h->use_traces || !(h->cfg.physics == DG_EULER && h->cfg.p >= 4);
+}
+// ... and close each step inside the next one's first stage
+static bool small_fold(const dg_handle *h) {
+  return small_path(h) && small_blocks(h->cfg.p, h->K) <= kSmallFold;
+}
+
 static StageArgs base_args(dg_handle *h) {
   StageArgs a;
   std::memset(&a, 0, sizeof a);
@@ -696,6 +710,7 @@ static StageArgs base_args(dg_handle *h) {
   a.bad = h->d_bad;  // valid always; used only where flags_in / flags_out say so
   a.vol_mfma = volume_mfma(h->cfg) ? 1 : 0;
   a.fired = h->d_fired;
+  a.small = small_path(h) ? 1 : 0;
   return a;
 }
 
@@ -728,9 +743,12 @@ static void refresh_bnd_fixed(dg_handle *h, double t) {
 
 // one stage launch, preceded by the boundary data at the stage time when needed
 static void launch_stage_bnd(dg_handle *h, const StageArgs &a) {
-  if (bnd_time_dependent(h))
+  // (the point-parallel stage evaluates it where it is used)
+  StageArgs s = a;
+  s.tdb = bnd_time_dependent(h) ? 1 : 0;
+  if (s.tdb && !s.small)
     launch_bnd(h->cfg.physics, h->cfg.p, a.m, h->ph, h->d_st, a.cstage, 1, 0., h->stream);
-  launch_stage(h->cfg.physics, h->cfg.p, a, h->stream);
+  launch_stage(h->cfg.physics, h->cfg.p, s, h->stream);
 }
 
 extern "C" int dg_eval_rhs(dg_handle *h, const double *u, double t, double dt, double *k,
@@ -933,7 +951,13 @@ static int build_step_io(dg_handle *h, StageArgs *st, int cfl_mode, double *cons
                          double *acc, bool conv = false) {
   StageArgs a = base_args(h);
   a.cfl_mode = cfl_mode;
-  return make_stages(a, h->cfg.integrator, posfix_on(h) ? 1 : 0, st, io, acc, conv);
+  const int n = make_stages(a, h->cfg.integrator, posfix_on(h) ? 1 : 0, st, io, acc, conv);
+  for (int q = 0; q < n; q++) {
+    st[q].conv_run = conv ? 1 : 0;
+    if (small_fold(h))
+      st[q].step_pos = q == 0 ? STEP_FIRST : (q == n - 1 ? STEP_LAST : STEP_MID);
+  }
+  return n;
 }
 
 static int nstages_of(int integ) {
@@ -945,7 +969,7 @@ static int nstages_of(int integ) {
 // unless DG_STAGE_GATHER is set in the environment when the handle is
 // created (then every stage gathers the neighbours' modes).
 static bool traces_wanted(const dg_handle *h) {
-  return h->use_traces && h->cfg.physics == DG_EULER && h->cfg.p >= 4 &&
+  return h->use_traces && !small_path(h) && h->cfg.physics == DG_EULER && h->cfg.p >= 4 &&
          (long long)tr_elem(h->cfg.p) * h->K < (1ll << 28);
 }
 
@@ -1081,7 +1105,18 @@ static int run_steps(dg_handle *h, int max_steps, double fixed_dt, double t_end,
   HIPCHK(h, hipGetLastError());
   DevState hs;
   std::memset(&hs, 0, sizeof hs);
+  // (a small-mesh run leaves its last step to be closed here)
+  const bool fold = !h->cfg.limiter && small_fold(h);
   auto read_state = [&]() -> int {
+    if (fold) {
+      FinishArgs f{};
+      f.cfl_mode = cfl_mode;
+      f.cfl_num = h->cfg.cfl * h->min_r;
+      f.p = p;
+      f.conv = conv ? 1 : 0;
+      f.if_pending = 1;
+      launch_finish(h->d_st, h->d_part, small_blocks(p, h->K), f, h->stream);
+    }
     HIPCHK(h, hipMemcpyAsync(&hs, h->d_st, sizeof hs, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return DG_OK;

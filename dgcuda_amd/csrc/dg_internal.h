@@ -50,10 +50,17 @@ struct DevState {
   double conv;                  // last reduced step-to-step change
   int halt;                     // 1: t_end reached, 2: converged; every stage launch then exits
   int steps;                    // steps completed since the state was written
+  int pending;                  // small meshes: the last step's maxima wait in the partials
 };
 
 enum StageMode { M_KONLY = 0, M_US_CK = 1, M_A_UN_B_US_CK = 2, M_UN_CK = 3 };
 enum AccMode { ACC_NONE = 0, ACC_SET6 = 1, ACC_ADD3 = 2, ACC_FINAL6 = 3 };
+
+// where a small-mesh stage stands in its step (k_stage_s); STEP_NONE: the
+// step is closed by a launch of its own (or there is none)
+enum StepPos { STEP_NONE = 0, STEP_FIRST = 1, STEP_MID = 2, STEP_LAST = 3 };
+// blocks whose partials the first stage of a small-mesh step reduces itself
+constexpr int kSmallFold = 1024;
 
 struct MeshDev {
   int K;
@@ -112,6 +119,10 @@ struct StageArgs {
   // tr_out: written for the stage's output
   const double *tr_in;
   double *tr_out;
+  // small meshes: the point-parallel stage (k_stage_s), its place in the
+  // step, whether the run reduces the step-to-step change, and whether its
+  // side points evaluate time-dependent boundary data
+  int small, step_pos, conv_run, tdb;
   int *fired;  // set to 1 wherever the positivity fix fires or a stored state is flagged
 };
 
@@ -127,6 +138,7 @@ struct FinishArgs {
   int initial;      // 1: before the first step (no step completed)
   double t0;        // time of the initial state
   int conv;         // 1: the partials hold the step-to-step change too
+  int if_pending;   // 1: only a state marked pending has a step to close
 };
 
 // ensemble (dg_ensemble.hip): group p of the merged mesh runs blocks
@@ -167,6 +179,8 @@ void launch_set_state(DevState *st, double t, double dt, hipStream_t s);
 // launchers (dg_kernels.hip)
 int upload_tables(int p, const void *tab, size_t bytes);
 void launch_stage(int phys, int p, const StageArgs &a, hipStream_t s);
+int small_max_k(int phys, int p);      // largest mesh of the point-parallel stage
+int small_blocks(int p, int K);        // its blocks
 void launch_init(int phys, int p, const MeshDev &m, const PhysParams &ph, double *c, hipStream_t s);
 // per-element error integrals (norm 1 or 2), [N][K]
 void launch_err(int phys, int p, int norm, const MeshDev &m, const PhysParams &ph,

@@ -32,6 +32,7 @@
 #include "dg_device.h"
 #include "dg_stage.h"
 #include "dg_stage_q.h"
+#include "dg_stage_s.h"
 
 namespace dgk {
 
@@ -119,10 +120,44 @@ __global__ __launch_bounds__((stage_blk<PHYS, P>())) void k_stage(const StageArg
   stage_body<PHYS, P, B>(a, blockIdx.x, a.nblk, s_side, s_c);
 }
 
+int small_blocks(int p, int K) { return nblocks(K, small_eb(p)); }
+
+// The point-parallel stage (dg_stage_s.h) up to these many elements.  Below,
+// the one-thread (or four-lane) stage costs the instruction stream of a
+// single wave whatever the mesh: us per SSP-RK3 stage, the step's close
+// included, periodic meshes, point-parallel against the wide kernel:
+//   Euler p = 3    968: 8.1 / 32    8,192: 13.1 / 20.6   16,200: 22.2 / 20.9
+//   Euler p = 4    968: 10 / 33     4,050: 13 / 32        8,192: 18.2 / 17.5
+//   SWE Roe p = 3  968: 6.2 / 17   16,200: 16.9 / 17.8   32,768: 27.9 / 18.8
+//   TE p = 5       968: 7.4 / 76   16,200: 41 / 69       32,768: 77 / 71
+//   adv p = 1      968: 4.0 / 5.0   8,192: 4.5 / 5.0     16,200: 5.4 / 5.1
+// Above, the LDS table reads per multiply-add set its time (1.25 per
+// multiply-add with four variables, more with fewer), which the wide kernels
+// do not have.
+int small_max_k(int phys, int p) {
+  static constexpr int k[3][PMAX + 1] = {{32768, 12288, 16384, 12288, 12288, 8192},
+                                         {32768, 16384, 16384, 16384, 20480, 28672},
+                                         {16384, 12288, 16384, 14336, 6144, 6144}};
+  const int n = nvars_of(phys);
+  return k[n == 1 ? 0 : n - 2][p];
+}
+
 void launch_stage(int phys, int p, const StageArgs &a0, hipStream_t s) {
   StageArgs a = a0;
   dispatch(phys, p, [&](auto PH, auto PP) {
     constexpr int ph = decltype(PH)::value, pp = decltype(PP)::value;
+    if (a.small) {
+      a.nblk = small_blocks(pp, a.m.K);
+      const dim3 g(a.nblk), b(kSmallT);
+      if constexpr (small_tdb<ph>()) {
+        if (a.tdb) {
+          hipLaunchKernelGGL((k_stage_s<ph, pp, true>), g, b, 0, s, a);
+          return;
+        }
+      }
+      hipLaunchKernelGGL((k_stage_s<ph, pp, false>), g, b, 0, s, a);
+      return;
+    }
     if constexpr (stage_quad<ph, pp>()) {
       a.nblk = nblocks(a.m.K, kQuadBlk / 4);
       const dim3 g(a.nblk), b(kQuadBlk);
@@ -146,7 +181,7 @@ void launch_stage(int phys, int p, const StageArgs &a0, hipStream_t s) {
       hipLaunchKernelGGL((k_stage<ph, pp>), dim3(a.nblk), dim3(B), 0, s, a);
     }
   });
-  if (a.last_stage) {
+  if (a.last_stage && a.step_pos == STEP_NONE) {
     FinishArgs f{};
     f.cfl_mode = a.cfl_mode;
     f.cfl_num = a.cfl_num;

@@ -97,6 +97,23 @@ constexpr double phi_bound(int i) {
   return m;
 }
 
+// whether states within mean +- dev keep the density (and for Euler the
+// pressure) positive with a wide margin over rounding
+template <int PHYS>
+__device__ __forceinline__ bool bounds_physical(const double *mean, const double *dev) {
+  constexpr double margin = 1e-10;
+  const double rmin = mean[0] - dev[0];
+  const double rsc = fabs(mean[0]) + dev[0];
+  if (!(rmin > margin * rsc)) return false;
+  if constexpr (PHYS == PH_EULER) {
+    const double mx = fabs(mean[1]) + dev[1], my = fabs(mean[2]) + dev[2];
+    const double emin = mean[3] - dev[3];
+    const double kin = 0.5 * (mx * mx + my * my) * frcp(rmin);
+    return emin - kin > margin * (fabs(mean[3]) + dev[3] + kin);
+  }
+  return true;
+}
+
 // Sufficient condition for elem_physical: every point value lies within
 // mean +- sum_i |c_i| max|phi_i|; if those bounds keep the density (and for
 // Euler the pressure) positive with a wide margin over rounding, every point
@@ -115,16 +132,7 @@ __device__ __forceinline__ bool surely_physical(const PhysParams &ph,
     for (int i = 1; i < NP; i++) d = fma(fabs(o[n][i]), phi_bound<P>(i), d);
     dev[n] = d * (1. + margin);
   }
-  const double rmin = mean[0] - dev[0];
-  const double rsc = fabs(mean[0]) + dev[0];
-  if (!(rmin > margin * rsc)) return false;
-  if constexpr (PHYS == PH_EULER) {
-    const double mx = fabs(mean[1]) + dev[1], my = fabs(mean[2]) + dev[2];
-    const double emin = mean[3] - dev[3];
-    const double kin = 0.5 * (mx * mx + my * my) * frcp(rmin);
-    return emin - kin > margin * (fabs(mean[3]) + dev[3] + kin);
-  }
-  return true;
+  return bounds_physical<PHYS>(mean, dev);
 }
 
 // the point check itself (check_physical's test at every volume and side
@@ -670,13 +678,50 @@ __device__ __forceinline__ void stage_body(const StageArgs a, int pblock, int nb
   }
 }
 
+// Closing a step from its maxima: dt of the next step from the CFL rule
+// (time_integrator.cu:217) or kept, time bookkeeping (:226-231), the NaN
+// guard (:219-223), the stop at t_end with the last dt shortened to land on
+// it (:225-228) and the convergence stop (:403-417).  `initial` marks the
+// call before the first step, which starts at t0.
+__device__ __forceinline__ void close_step(DevState &S, double lmax, double cv,
+                                           const FinishArgs &f, double t0) {
+  double dtn;
+  if (f.cfl_mode)
+    dtn = f.cfl_num / lmax / (2. * f.p + 1.);
+  else
+    dtn = f.initial ? f.fixed_dt : S.dt;
+  if (f.initial) {
+    S.tdone = t0;
+    S.dt_last = 0.;
+    if (S.conv_tol >= 0.) {  // the reference starts from conv = 1 (time_integrator.cu:193)
+      S.conv = 1.;
+      if (!(1. > S.conv_tol)) S.halt = 2;
+    }
+  } else {
+    S.tdone = S.t;
+    S.dt_last = S.dt;
+    S.steps += 1;
+  }
+  S.lam_max = lmax;
+  if (dtn != dtn) S.nan_flag = 1;
+  if (f.conv) {
+    S.conv = cv;
+    if (!(cv > S.conv_tol)) S.halt = 2;
+  }
+  double tn = S.tdone + dtn;
+  if (S.tdone >= S.t_end) {
+    S.halt = 1;
+  } else if (tn > S.t_end) {
+    dtn = S.t_end - S.tdone;
+    tn = S.t_end;
+  }
+  S.dt = dtn;
+  S.t = tn;
+}
+
 // Step reduction, part 2 (one block): the max over the partials closes the
-// step: dt of the next step from the CFL rule (time_integrator.cu:217) or
-// kept, time bookkeeping (time_integrator.cu:226-231), the NaN guard
-// (:219-223), the stop at t_end with the last dt shortened to land on it
-// (:225-228) and the convergence stop (:403-417).  `initial` marks the call
-// before the first step, which starts at t0.  pl / pc: the nblk partial keys
-// of the CFL speed and of the step-to-step change (pc: nullptr without it).
+// step.  pl / pc: the nblk partial keys of the CFL speed and of the
+// step-to-step change (pc: nullptr without it).
 __device__ __forceinline__ void finish_body(DevState *st, const unsigned long long *pl,
                                             const unsigned long long *pc, int nblk,
                                             const FinishArgs &f, double t0) {
@@ -723,40 +768,9 @@ __device__ __forceinline__ void finish_body(DevState *st, const unsigned long lo
     s_c[0] = s_c[w] > s_c[0] ? s_c[w] : s_c[0];
   }
   if (S.nan_flag | S.halt) return;
-  const double lmax = ord_val(s_l[0]);
-  double dtn;
-  if (f.cfl_mode)
-    dtn = f.cfl_num / lmax / (2. * f.p + 1.);
-  else
-    dtn = f.initial ? f.fixed_dt : S.dt;
-  if (f.initial) {
-    S.tdone = t0;
-    S.dt_last = 0.;
-    if (S.conv_tol >= 0.) {  // the reference starts from conv = 1 (time_integrator.cu:193)
-      S.conv = 1.;
-      if (!(1. > S.conv_tol)) S.halt = 2;
-    }
-  } else {
-    S.tdone = S.t;
-    S.dt_last = S.dt;
-    S.steps += 1;
-  }
-  S.lam_max = lmax;
-  if (dtn != dtn) S.nan_flag = 1;
-  if (f.conv) {
-    const double cv = ord_val(s_c[0]);
-    S.conv = cv;
-    if (!(cv > S.conv_tol)) S.halt = 2;
-  }
-  double tn = S.tdone + dtn;
-  if (S.tdone >= S.t_end) {
-    S.halt = 1;
-  } else if (tn > S.t_end) {
-    dtn = S.t_end - S.tdone;
-    tn = S.t_end;
-  }
-  S.dt = dtn;
-  S.t = tn;
+  if (f.if_pending && !S.pending) return;
+  S.pending = 0;
+  close_step(S, ord_val(s_l[0]), ord_val(s_c[0]), f, t0);
   *st = S;
 }
 

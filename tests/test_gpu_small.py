@@ -1,0 +1,87 @@
+"""The stage's two kernel families against the oracle on both sides of the
+mesh size that separates them: the point-parallel stage of small meshes (a
+thread per point; dg_stage_s.h) at its smallest and largest meshes, ragged
+against its 4 to 64 elements per block, closing its steps inside the next
+one's first stage (up to 1,024 blocks) or by a launch (above); and the
+one-thread and four-lane stages just above.  Both evaluate the same
+expressions as the oracle with other roundings: 1e-12 relative L2, the bar of
+the parity tests."""
+import numpy as np
+import pytest
+
+from dgcuda_amd import _lib as L
+from dgcuda_amd import mesh as M
+from tests.helpers import make_pair, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+MAX_K = {1: (32768, 12288, 16384, 12288, 12288, 8192),
+         3: (32768, 16384, 16384, 16384, 20480, 28672),
+         4: (16384, 12288, 16384, 14336, 6144, 6144)}  # by variables, order
+
+
+def _pair(physics, p, K, periodic, **kw):
+    nx = int(np.sqrt(K / 2))
+    mesh = M.structured(nx, (K // 2) // nx, periodic=periodic, jitter=0.2, seed=7)
+    eps = np.random.default_rng(3).uniform(1.0, 4.0, mesh.K)
+    s, o = make_pair(physics, p, mesh, eps_elem=eps if physics == L.MAXWELL_TE else None, **kw)
+    s.project_ic()
+    o.project_ic()
+    return s, o
+
+
+@pytest.mark.parametrize("physics", [L.ADVECTION, L.EULER, L.SWE, L.MAXWELL_TM, L.MAXWELL_TE])
+@pytest.mark.parametrize("p", [0, 1, 2, 3, 4, 5])
+def test_rhs_either_side_of_the_size_rule(physics, p):
+    top = MAX_K[L.NVARS[physics]][p]
+    for K in (18, top, top + 2 * int(np.sqrt(top))):
+        s, o = _pair(physics, p, K, periodic=False)
+        u = o.coeffs()
+        u = u * (1.0 + 0.05 * np.random.default_rng(p).standard_normal(u.shape))
+        if physics in (L.EULER, L.SWE):
+            u[:, 1:, ::41] *= 400.0  # elements that contribute their means only
+        print("physics", physics, "p", p, "K", s.K, flush=True)
+        r = rel_l2(s.eval_rhs(u, t=0.1, dt=0.01), o.eval_rhs(u, t=0.1, dt=0.01))
+        print("  rel", r)
+        assert r < TOL
+        s.close()
+
+
+@pytest.mark.parametrize("physics,p,K,integrator", [
+    (L.EULER, 1, 11250, L.RK4), (L.EULER, 4, 6100, L.SSPRK3), (L.EULER, 4, 6498, L.SSPRK3),
+    (L.EULER, 5, 6498, L.RK4), (L.EULER, 3, 14450, L.RK2MID), (L.SWE, 4, 18432, L.SSPRK3),
+    (L.SWE, 4, 8190, L.SSPRK2), (L.MAXWELL_TE, 5, 8450, L.RK4), (L.ADVECTION, 0, 31250, L.SSPRK3)])
+def test_steps_either_side_of_the_size_rule(physics, p, K, integrator):
+    s, o = _pair(physics, p, K, periodic=True, integrator=integrator, cfl=0.2)
+    print("physics", physics, "p", p, "K", s.K, flush=True)
+    ts, dts = s.step(5)  # graphs of 4 and 1 steps
+    rc, to, dto = o.run(5)
+    r = rel_l2(s.coeffs(), o.coeffs())
+    print("  rel", r, "t", ts, to)
+    assert rc == 0 and abs(ts - to) <= 1e-13 * to and abs(dts - dto) <= 1e-13 * dto
+    assert r < TOL
+    s.close()
+
+
+def test_stops_and_time_dependent_boundaries_on_a_small_mesh():
+    """t_end, the step-to-step change and a moving inflow in one run: the
+    steps taken, the time reached and the state are the oracle's"""
+    mesh = M.structured(9, 11, lx=2.0, ly=2.0, x0=-1.0, y0=-1.0, periodic=False, jitter=0.2,
+                        seed=3, bc=(-3, -3, -2, -3))
+    s, o = make_pair(L.ADVECTION, 3, mesh, problem=L.PROB_ADV_ROTHILL, params=())
+    s.project_ic()
+    o.project_ic()
+    print("hill", s.K, flush=True)
+    t, dt = s.step(6)
+    rc, to, _ = o.run(6)
+    assert rc == 0 and abs(t - to) <= 1e-13 * to and rel_l2(s.coeffs(), o.coeffs()) < TOL
+    # t_end (the third step is shortened), then the change of the first step
+    # (the reference starts its convergence loop from a change of 1)
+    for kw in (dict(t_end=t + 2.5 * dt), dict(max_steps=50, conv_tol=0.9)):
+        t, n, c = s.run(t=t, **kw)
+        rc, to, no, co, _ = o.run_until(t0=to, **kw)
+        assert rc == 0 and n == no and abs(t - to) <= 1e-13 * to
+        assert rel_l2(s.coeffs(), o.coeffs()) < TOL
+        assert "conv_tol" not in kw or abs(c - co) <= 1e-12 * abs(co)
+    s.close()
