@@ -323,6 +323,10 @@ __host__ __device__ constexpr bool linear_flux() {
   return PHYS == PH_ADV || PHYS == PH_TM || PHYS == PH_TE;
 }
 
+}  // namespace dgk
+#include "dg_vjp_s.h"
+namespace dgk {
+
 // MODE 1: (dk/du)^T lam, reading the state.  For the linear systems the
 // transpose does not read the state: MODE 0 computes it without.
 // The element's own weights (and state, where read) wait in LDS while its
@@ -1079,9 +1083,40 @@ __global__ __launch_bounds__(BLK) void k_combine(const CombArgs c) {
   gst_nt(c.out + q, e, v);
 }
 
+// The point-parallel VJP (dg_vjp_s.h) up to these many elements, by system
+// (the last row: TE with the permittivity gradient) and order.  As for the
+// stage, the wide kernels cost one wave's code below, and LDS reads bound the
+// point-parallel one above: us per stage of a reverse sweep (recompute
+// included), point-parallel against wide, on 968 / 8,192 / 32,768 elements:
+//   Euler p = 3    20 / 92    48 / 93    168 / 143
+//   Euler p = 4    25 / 41    65 / 60    226 / 133
+//   SWE Roe p = 3  17 / 79    31 / 79     90 / 105
+//   TM p = 5       18 / 133   53 / 151   172 / 257
+//   TE eps p = 3   16 / 35    30 / 42     89 / 61
+//   adv p = 1      12 / 13    12 / 13     17 / 15
+static int small_max_vjp(int phys, int p, bool eps) {
+  static constexpr int k[5][PMAX + 1] = {{32768, 12288, 16384, 16384, 16384, 10240},
+                                         {32768, 24576, 20480, 20480, 6144, 4096},
+                                         {32768, 24576, 24576, 40960, 28672, 20480},
+                                         {32768, 16384, 32768, 24576, 65536, 65536},
+                                         {40960, 24576, 20480, 14336, 14336, 14336}};
+  return k[phys == PH_TE ? (eps ? 4 : 3) : phys][p];
+}
+
 void launch_adjoint_rhs(int phys, int p, const AdjArgs &a, hipStream_t s) {
   dispatch(phys, p, [&](auto PH, auto PP) {
     constexpr int ph = decltype(PH)::value, pp = decltype(PP)::value;
+    if (a.m.K <= small_max_vjp(ph, pp, a.geps != nullptr)) {
+      const dim3 g(nblocks(a.m.K, small_eb(pp))), b(kSmallT);
+      if constexpr (ph == PH_TE) {
+        if (a.geps) {
+          hipLaunchKernelGGL((k_vjp_s<ph, pp, true>), g, b, 0, s, a);
+          return;
+        }
+      }
+      hipLaunchKernelGGL((k_vjp_s<ph, pp, false>), g, b, 0, s, a);
+      return;
+    }
     auto go = [&](auto M) {
       constexpr int md = decltype(M)::value, B = vjp_blk<ph, pp, md>();
       hipLaunchKernelGGL((k_vjp<ph, pp, md>), dim3(nblocks(a.m.K, B)), dim3(B), 0, s, a);

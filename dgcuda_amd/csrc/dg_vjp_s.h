@@ -1,0 +1,258 @@
+// dg_vjp_s.h -- the right-hand side's vector-Jacobian product on small
+// meshes: a thread per point, then a thread per coefficient, as the small
+// mesh stage (dg_stage_s.h).  One launch does what the wide path does in up
+// to three: for Maxwell TE's permittivity gradient the side points also form
+// the impedance terms (k_eps_side), and for Euler p >= 4 the epilogue adds
+// the Runge-Kutta terms itself (k_combine), the registers being free here.
+// Included by dg_adjoint.hip (the flux VJPs it uses are defined there).
+#pragma once
+
+#include "dg_stage_s.h"
+
+namespace dgk {
+
+template <int PHYS, int P, bool EPS>
+__global__ __launch_bounds__(kSmallT) void k_vjp_s(const AdjArgs a) {
+  using TC = TabC<P>;
+  constexpr int NP = TC::NP, NQ = TC::NQ, NQ1 = TC::NQ1, N = nvars_of(PHYS);
+  constexpr bool TE = PHYS == PH_TE;
+  constexpr bool kU = EPS || !linear_flux<PHYS>();  // the state is read
+  constexpr int EB = small_eb(P), NR = N * NP, NS = 3 * NQ1, T = kSmallT;
+  constexpr int RW = T / EB, R = (NR + RW - 1) / RW, RN = (3 * NR + RW - 1) / RW;
+  constexpr int RU = kU ? NR : 1;
+  __shared__ double s_B[NP * NQ], s_GX[NP * NQ], s_GY[NP * NQ], s_side[3 * NP * NQ1];
+  __shared__ double s_w[NR][EB], s_nw[3 * NR][EB], s_u[RU][EB], s_nu[3 * RU][EB];
+  __shared__ double s_f[NS][N][EB], s_g[NQ][N][EB];
+  __shared__ double s_z[EPS ? NS : 1][EB], s_k[EPS ? 2 * NP : 1][EB];
+  const int t = threadIdx.x, el = t % EB, row = t / EB;
+  const int K = a.m.K;
+  const int e = remap_block(blockIdx.x, (K + EB - 1) / EB) * EB + el;
+  const bool act = e < K;
+  const int ee = act ? e : K - 1;
+
+  // ---- loads
+  int nbq[RN];
+#pragma unroll
+  for (int q = 0; q < RN; q++) {
+    const int r = row + q * RW, rr = r < 3 * NR ? r : 0;
+    nbq[q] = a.m.slot[(size_t)(rr / NR) * K + ee].x;
+  }
+  const bool is_side = t < EB * NS, is_vol = !is_side && t < EB * (NS + NQ);
+  const int sp = is_side ? row : 0, sk = sp / NQ1, jj = sp - sk * NQ1;
+  const int vj = is_vol ? row - NS : 0;
+  const int2 sl = a.m.slot[(size_t)sk * K + ee];
+  double ow[R], ou[R];
+#pragma unroll
+  for (int q = 0; q < R; q++) {
+    const int r = row + q * RW, rr = r < NR ? r : 0;
+    ow[q] = gld(a.lam + (size_t)rr * K, ee);
+    ou[q] = 0.;
+    if constexpr (kU) ou[q] = gld(a.us + (size_t)rr * K, ee);
+  }
+  const double xr = gld(a.m.xr, ee), yr = gld(a.m.yr, ee);
+  const double xs = gld(a.m.xs, ee), ys = gld(a.m.ys, ee);
+  const double Jme = gld(a.m.J, ee);
+  double eps_me = 1., eps_nb = 1.;
+  if constexpr (TE) eps_me = gld(a.m.eps, ee);
+  double Vv[6] = {0., 0., 0., 0., 0., 0.};
+  const bool vary = PHYS == PH_ADV && a.ph.prob == PB_ADV_ROTHILL;
+  if (vary) {
+#pragma unroll
+    for (int q = 0; q < 6; q++) Vv[q] = gld(a.m.V + (size_t)q * K, ee);
+  }
+  for (int q = t; q < NP * NQ; q += T) {
+    s_B[q] = TC::B[q];
+    s_GX[q] = TC::GX[q];
+    s_GY[q] = TC::GY[q];
+  }
+  for (int q = t; q < 3 * NP * NQ1; q += T) s_side[q] = TC::SIDE[q];
+#pragma unroll
+  for (int q = 0; q < RN; q++) {
+    const int r = row + q * RW;
+    if (r < 3 * NR) {
+      const bool has = nbq[q] >= 0;
+      const int nb = has ? nbq[q] : ee;
+      const double w = gld(a.lam + (size_t)(r % NR) * K, nb);
+      s_nw[r][el] = has ? w : 0.;
+      if constexpr (kU) {
+        const double u = gld(a.us + (size_t)(r % NR) * K, nb);
+        s_nu[r][el] = has ? u : 0.;
+      }
+    }
+  }
+  double nx = 0., ny = 0., len = 0., Jnb = 1., bv[NMAX] = {0., 0., 0., 0.};
+  if (is_side) {
+    const int sid = sl.y >> 3;
+    nx = gld(a.m.snx, sid);
+    ny = gld(a.m.sny, sid);
+    len = gld(a.m.slen, sid);
+    Jnb = gld(a.m.J, sl.x >= 0 ? sl.x : ee);
+    if constexpr (TE) eps_nb = sl.x >= 0 ? gld(a.m.eps, sl.x) : eps_me;
+    if (sl.x < 0) {
+      const double *b = a.m.bnd_val + ((size_t)a.m.side[sid].w * NQ1 + jj) * NMAX;
+#pragma unroll
+      for (int n = 0; n < NMAX; n++) bv[n] = b[n];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < R; q++) {
+    const int r = row + q * RW;
+    if (r < NR) {
+      s_w[r][el] = ow[q];
+      if constexpr (kU) s_u[r][el] = ou[q];
+    }
+  }
+  // the weights' scale dt / J (TE also 1/eps, 1/mu per row), times lc
+  const double sme = a.lc * (a.dt / Jme);
+  auto scale = [&](double s, double eps, int n) {
+    if constexpr (TE) return s * (n < 2 ? 1. / eps : 1. / a.ph.mu);
+    return s;
+  };
+  __syncthreads();
+
+  // ---- points
+  if (is_side) {
+    const int nb = sl.x, nbls = sl.y & 3, role = (sl.y >> 2) & 1;
+    const double *po = s_side + (size_t)(sk * NP) * NQ1 + jj;
+    const double *pn = s_side + (size_t)(nbls * NP) * NQ1 + NQ1 - 1 - jj;
+    double Um[NMAX] = {0., 0., 0., 0.}, Un[NMAX] = {0., 0., 0., 0.}, Wm[N], Wn[N];
+#pragma unroll
+    for (int n = 0; n < N; n++) Wm[n] = Wn[n] = 0.;
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+      const double x = po[i * NQ1], y = pn[i * NQ1];
+#pragma unroll
+      for (int n = 0; n < N; n++) {
+        Wm[n] = fma(s_w[n * NP + i][el], x, Wm[n]);
+        Wn[n] = fma(s_nw[sk * NR + n * NP + i][el], y, Wn[n]);
+        if constexpr (kU) {
+          Um[n] = fma(s_u[n * NP + i][el], x, Um[n]);
+          Un[n] = fma(s_nu[sk * NR + n * NP + i][el], y, Un[n]);
+        }
+      }
+    }
+    if constexpr (kU) {
+      if (nb == -1) {
+        wall_state<PHYS>(a.ph, Um, Un, bv[0], bv[1], bv[2]);
+      } else if (nb < 0) {
+#pragma unroll
+        for (int n = 0; n < N; n++) Un[n] = bv[n];
+      }
+    }
+    const double snb = a.lc * (a.dt / Jnb);
+    const double f = (role ? 0.5 : -0.5) * len * TC::W1[jj];
+    double UL[NMAX], UR[NMAX], gF[NMAX] = {0., 0., 0., 0.}, gL[NMAX] = {0., 0., 0., 0.},
+                               gR[NMAX] = {0., 0., 0., 0.};
+#pragma unroll
+    for (int n = 0; n < NMAX; n++) {
+      UL[n] = role ? Un[n] : Um[n];
+      UR[n] = role ? Um[n] : Un[n];
+    }
+#pragma unroll
+    for (int n = 0; n < N; n++)
+      gF[n] = f * (scale(sme, eps_me, n) * Wm[n] - scale(snb, eps_nb, n) * Wn[n]);
+    PhysParams pv = a.ph;
+    if constexpr (PHYS == PH_ADV) {
+      if (vary) {
+        double x, y;
+        side_point<NQ1>(Vv, TC::X1, sk, jj, x, y);
+        rothill_velocity(x, y, pv.ax, pv.ay);
+      }
+    }
+    double gzl, gzr;
+    riemann_vjp<PHYS>(pv, UL, UR, nx, ny, role ? eps_nb : eps_me, role ? eps_me : eps_nb, gF, gL,
+                      gR, gzl, gzr);
+    double gme[NMAX];
+#pragma unroll
+    for (int n = 0; n < N; n++) gme[n] = role ? gR[n] : gL[n];
+    if (nb == -1) wall_vjp<PHYS>(a.ph, bv[0], bv[1], bv[2], gR, gme);
+#pragma unroll
+    for (int n = 0; n < N; n++) s_f[sp][n][el] = gme[n];
+    // a boundary's ghost state carries the element's own impedance
+    if constexpr (EPS) s_z[sp][el] = nb < 0 ? gzl + gzr : (role ? gzr : gzl);
+  } else if (is_vol) {
+    double U[NMAX] = {0., 0., 0., 0.}, gfx[NMAX], gfy[NMAX], gU[NMAX] = {0., 0., 0., 0.};
+    double wa[N], wb[N];
+#pragma unroll
+    for (int n = 0; n < N; n++) wa[n] = wb[n] = 0.;
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+      const double gx = s_GX[i * NQ + vj], gy = s_GY[i * NQ + vj], ph = s_B[i * NQ + vj];
+#pragma unroll
+      for (int n = 0; n < N; n++) {
+        wa[n] = fma(s_w[n * NP + i][el], gx, wa[n]);
+        wb[n] = fma(s_w[n * NP + i][el], gy, wb[n]);
+        if constexpr (kU) U[n] = fma(s_u[n * NP + i][el], ph, U[n]);
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+      const double sc = scale(sme, eps_me, n);
+      gfx[n] = sc * (wa[n] * ys - wb[n] * yr);
+      gfy[n] = sc * (wb[n] * xr - wa[n] * xs);
+    }
+    PhysParams pv = a.ph;
+    if constexpr (PHYS == PH_ADV) {
+      if (vary) {
+        double x, y;
+        elem_point(Vv, TC::R1[vj], TC::R2[vj], x, y);
+        rothill_velocity(x, y, pv.ax, pv.ay);
+      }
+    }
+    fn_vjp<PHYS>(pv, U, 1.0, 0.0, gfx, gU);
+    fn_vjp<PHYS>(pv, U, 0.0, 1.0, gfy, gU);
+#pragma unroll
+    for (int n = 0; n < N; n++) s_g[vj][n][el] = gU[n];
+  }
+  __syncthreads();
+
+  // ---- modes
+#pragma unroll
+  for (int q = 0; q < R; q++) {
+    const int r = row + q * RW;
+    if (r < NR) {
+      const int n = r / NP, i = r % NP;
+      const size_t o = (size_t)r * K;
+      // the combination arrays first: they are in flight during the sums
+      double x[4], y[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        x[u] = a.gout && u < a.nout ? gld(a.ot[u] + o, ee) : 0.;
+        y[u] = a.gout2 && u < a.n2 ? gld(a.o2t[u] + o, ee) : 0.;
+      }
+      double g = 0.;
+#pragma unroll
+      for (int j = 0; j < NQ; j++) g = fma(s_g[j][n][el], s_B[i * NQ + j], g);
+#pragma unroll
+      for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int j = 0; j < NQ1; j++)
+          g = fma(s_f[k * NQ1 + j][n][el], s_side[(k * NP + i) * NQ1 + j], g);
+      double v = a.scale * g, v2 = a.c2g * g;
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        if (u < a.nout) v = fma(a.oc[u], x[u], v);
+        if (u < a.n2) v2 = fma(a.o2c[u], y[u], v2);
+      }
+      if (act && a.gout) gst(a.gout + o, e, v);
+      if (act && a.gout2) gst(a.gout2 + o, e, v2);
+      if constexpr (EPS) {
+        if (n < 2) s_k[r][el] = ow[q] * gld(a.kst + o, ee);
+      }
+    }
+  }
+  if constexpr (EPS) {
+    __syncthreads();
+    if (row == 0 && act) {
+      // dz/deps = -z / (2 eps) on the sides, and the row scaling
+      // -lc lam . k_E / eps
+      double gz = 0., ew = 0.;
+      for (int s = 0; s < NS; s++) gz += s_z[s][el];
+      for (int r = 0; r < 2 * NP; r++) ew += s_k[r][el];
+      const double z = sqrt(a.ph.mu / eps_me);
+      a.geps[e] += a.scale * (gz * (-z / (2. * eps_me)) - a.lc * ew / eps_me);
+    }
+  }
+}
+
+}  // namespace dgk

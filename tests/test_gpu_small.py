@@ -64,6 +64,58 @@ def test_steps_either_side_of_the_size_rule(physics, p, K, integrator):
     s.close()
 
 
+@pytest.mark.parametrize("physics,p,K", [
+    (L.EULER, 3, 20480), (L.EULER, 4, 6144), (L.EULER, 5, 4096), (L.SWE, 4, 28672),
+    (L.MAXWELL_TM, 2, 32768), (L.MAXWELL_TE, 3, 14336), (L.MAXWELL_TE, 5, 14336),
+    (L.ADVECTION, 1, 12288)])
+def test_vjp_either_side_of_the_size_rule(physics, p, K):
+    """<g, J v> = <J^T g, v> on walled meshes with the rule's sizes: J v is
+    the oracle's central difference along a unit v (step 1e-4: truncation
+    ~1e-8 of a smooth second derivative, rounding ~1e-12)"""
+    for n in (18, K, K + 2 * int(np.sqrt(K))):
+        s, o = _pair(physics, p, n, periodic=False)
+        r = np.random.default_rng(p)
+        u = o.coeffs()
+        u = u + 0.01 * r.standard_normal(u.shape) / np.sqrt(u.shape[1])
+        v, g = r.standard_normal(u.shape), r.standard_normal(u.shape)
+        v /= np.linalg.norm(v)
+        h = 1e-4
+        fd = np.vdot(g, o.eval_rhs(u + h * v, dt=0.01) - o.eval_rhs(u - h * v, dt=0.01)) / (2 * h)
+        print("physics", physics, "p", p, "K", s.K, flush=True)
+        gu = s.adjoint_rhs(u, g, dt=0.01)
+        scale = np.linalg.norm(gu)
+        print("  fd", fd, "vjp", np.vdot(gu, v), "scale", scale)
+        assert abs(np.vdot(gu, v) - fd) < 1e-6 * scale
+        s.close()
+
+
+def test_eps_gradient_either_side_of_the_size_rule():
+    """the point-parallel VJP forms the impedance terms of dJ/deps itself, the
+    wide path (here 14,792 triangles) in a launch per side; each gradient
+    against central differences along one direction (step 1e-4)"""
+    for n in (7, 86):
+        mesh = M.structured(n, periodic=False, jitter=0.2, seed=5)
+        eps = np.random.default_rng(2).uniform(1.0, 4.0, mesh.K)
+        s, o = make_pair(L.MAXWELL_TE, 3, mesh, eps_elem=eps)
+        s.project_ic()
+        u0 = s.coeffs()
+        s.set_objective(L.OBJ_LINEAR, weights=np.random.default_rng(4).standard_normal(u0.shape))
+        dt = 0.2 / n / 7
+        print("eps gradient K", s.K, flush=True)
+        _, _, ge = s.adjoint_solve(3, dt, want_eps=True)
+        d = np.random.default_rng(6).standard_normal(mesh.K)
+        J = []
+        for h in (1e-4, -1e-4):
+            s.set_eps(eps + h * d)
+            s.set_coeffs(u0)
+            s.step(3, dt=dt)
+            J.append(s.objective())
+        fd = (J[0] - J[1]) / 2e-4
+        print("  fd", fd, "grad", ge @ d, "scale", np.linalg.norm(ge))
+        assert abs(ge @ d - fd) < 1e-6 * np.linalg.norm(ge) * np.linalg.norm(d)
+        s.close()
+
+
 def test_stops_and_time_dependent_boundaries_on_a_small_mesh():
     """t_end, the step-to-step change and a moving inflow in one run: the
     steps taken, the time reached and the state are the oracle's"""
