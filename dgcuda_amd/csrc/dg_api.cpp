@@ -65,9 +65,8 @@ struct dg_handle {
   // the first run of steps that uses them): views into d_trblk
   double *d_trblk = nullptr;
   double *d_tr[3] = {nullptr, nullptr, nullptr};
-  double *d_k[4] = {nullptr, nullptr, nullptr, nullptr};
+  double *d_k[2] = {nullptr, nullptr};
   double *d_err = nullptr, *d_lam = nullptr;
-  double *d_prev = nullptr;  // step base copy (convergence norm on the limiter path)
   DevState *d_st = nullptr;  // [2]: the state between steps, the running step's (k_stage_s)
   unsigned long long *d_part = nullptr;  // per-block maxima of the step reduction
   int *d_bad = nullptr;                  // positivity flags of the stored state d_c
@@ -358,7 +357,7 @@ static void free_mesh(dg_handle *h) {
   dfree(h->d_trblk);
   for (auto &t : h->d_tr) t = nullptr;
   for (auto &k : h->d_k) dfree(k);
-  dfree(h->d_err); dfree(h->d_lam); dfree(h->d_gw); dfree(h->d_prev); dfree(h->d_part); dfree(h->d_bad);
+  dfree(h->d_err); dfree(h->d_lam); dfree(h->d_gw); dfree(h->d_part); dfree(h->d_bad);
   drop_graphs(h);
   // no mesh from here until a new one is fully uploaded: every call that
   // needs one checks K, and the objective's weights went with the buffers
@@ -567,7 +566,8 @@ extern "C" int dg_set_mesh(dg_handle *h, int K, const double *V, const int *es, 
     h->d_acc = nv == 4 ? v[3] : nullptr;
   }
   if (h->cfg.limiter) {
-    int nk = h->cfg.integrator == DG_RK4 ? 4 : 1;
+    // the stage's k and (RK4) the running combination
+    int nk = h->cfg.integrator == DG_RK4 ? 2 : 1;
     for (int q = 0; q < nk; q++)
       if ((rc = alloc(h, (void **)&h->d_k[q], sb)) != DG_OK) return rc;
   }
@@ -1014,62 +1014,65 @@ static int build_step(dg_handle *h, StageArgs *st, int cfl_mode, bool conv = fal
   return ns;
 }
 
-// one step with separate launches and the limiter (the reference's order:
-// eval -> limit(k) -> tempstorage, ..., combine -> limit(c))
-static void limited_step(dg_handle *h, int cfl_mode, bool conv) {
-  const int phys = h->cfg.physics, p = h->cfg.p;
-  const long long n = (long long)dofs(h);
-  MeshDev m = mesh_dev(h);
-  StageArgs a = base_args(h);
-  a.mode = M_KONLY;
-  auto eval = [&](const double *us, double *k, double cst) {
-    StageArgs s = a;
-    s.us = us;
-    s.un = us;
-    s.out = k;
-    s.cstage = cst;
-    if (posfix_on(h)) launch_posfix(phys, p, h->K, h->ph, const_cast<double *>(us), h->stream);
+// One step with the limiter (the reference's order: eval -> limit(k) ->
+// tempstorage, ..., combine -> limit(c)): per stage the stage kernel stores k
+// and k_limited does the rest.  The new state goes to next: k_limited still
+// reads its neighbours' base means while others store.
+static void limited_step(dg_handle *h, int cfl_mode, bool conv, double *base, double *next) {
+  double *io[5];
+  const int S = nstages_of(h->cfg.integrator);
+  io[0] = base;
+  for (int s = 1; s < S; s++) io[s] = h->d_b1;
+  io[S] = next;
+  StageArgs a = base_args(h), st[4];
+  a.cfl_mode = cfl_mode;
+  a.conv_run = conv ? 1 : 0;
+  make_stages(a, h->cfg.integrator, 0, st, io, h->d_k[1], conv);
+  const int pf = posfix_on(h) ? 1 : 0;
+  const bool fold = small_fold(h);
+  for (int q = 0; q < S; q++) {
+    const StageArgs &r = st[q];
+    LimArgs l;
+    std::memset(&l, 0, sizeof l);
+    l.m = r.m;
+    l.ph = r.ph;
+    l.k = h->d_k[0];
+    l.un = base;
+    l.us = r.us;
+    l.acc = r.acc;
+    l.out = r.out;
+    l.st = fold ? h->d_st + 1 : h->d_st;
+    l.mode = r.mode;
+    l.accmode = r.accmode;
+    l.A = r.A;
+    l.B = r.B;
+    l.C = r.C;
+    l.final = r.last_stage;
+    l.fix = pf;
+    l.bad = h->d_bad;
+    l.conv = r.conv;
+    l.part = h->d_part;
+    l.small = small_path(h) ? 1 : 0;
+    l.nblk = limited_blocks(h->K, l.small);
+    StageArgs s = r;
+    s.out = h->d_k[0];
+    s.mode = M_KONLY;
+    s.accmode = ACC_NONE;
+    s.last_stage = s.conv = 0;
+    s.fix_in = q == 0 ? pf : 0;  // (the other inputs are stored fixed)
+    s.flags_in = pf;
+    if (fold) s.step_pos = q == 0 ? STEP_FIRST : (q == S - 1 ? STEP_LAST : STEP_MID);
     launch_stage_bnd(h, s);
-    launch_limit(phys, p, m, k, h->stream);
-  };
-  double *c = h->d_c, **k = h->d_k;
-  if (conv) launch_copy(n, h->d_prev, c, h->stream);
-  switch (h->cfg.integrator) {
-    case DG_RK4:
-      eval(c, k[0], 0.0);
-      launch_axpy(n, h->d_b1, c, 0.5, k[0], h->stream);
-      eval(h->d_b1, k[1], 0.5);
-      launch_axpy(n, h->d_b1, c, 0.5, k[1], h->stream);
-      eval(h->d_b1, k[2], 0.5);
-      launch_axpy(n, h->d_b1, c, 1.0, k[2], h->stream);
-      eval(h->d_b1, k[3], 1.0);
-      launch_rk4_final(n, c, k[0], k[1], k[2], k[3], h->stream);
-      break;
-    case DG_RK2MID:
-      eval(c, k[0], 0.0);
-      launch_axpy(n, h->d_b1, c, 0.5, k[0], h->stream);
-      eval(h->d_b1, k[0], 0.5);
-      launch_axpy(n, c, c, 1.0, k[0], h->stream);
-      break;
-    case DG_SSPRK2:
-      eval(c, k[0], 0.0);
-      launch_ssp(n, h->d_b1, nullptr, 0., c, 1., k[0], 1., h->stream);
-      eval(h->d_b1, k[0], 1.0);
-      launch_ssp(n, c, c, 0.5, h->d_b1, 0.5, k[0], 0.5, h->stream);
-      break;
-    case DG_SSPRK3:
-      eval(c, k[0], 0.0);
-      launch_ssp(n, h->d_b1, nullptr, 0., c, 1., k[0], 1., h->stream);
-      eval(h->d_b1, k[0], 1.0);
-      launch_ssp(n, h->d_b2, c, 0.75, h->d_b1, 0.25, k[0], 0.25, h->stream);
-      eval(h->d_b2, k[0], 0.5);
-      launch_ssp(n, c, c, 1. / 3., h->d_b2, 2. / 3., k[0], 2. / 3., h->stream);
-      break;
+    launch_limited(h->cfg.physics, l, h->stream);
+    if (l.final && !fold) {
+      FinishArgs f{};
+      f.cfl_mode = cfl_mode;
+      f.cfl_num = a.cfl_num;
+      f.p = h->cfg.p;
+      f.conv = l.conv;
+      launch_finish(h->d_st, h->d_part, l.nblk, f, h->stream);
+    }
   }
-  launch_limit(phys, p, m, c, h->stream);
-  // close the step: next dt from the limited state
-  launch_lambda_init(phys, p, m, h->ph, c, h->d_st, cfl_mode, h->cfg.cfl * h->min_r, 0., 0., 0,
-                     nullptr, h->stream, conv ? h->d_prev : nullptr, h->N, h->d_part);
 }
 
 // The time loop of time_integrate_rk4 / time_integrate_rk2
@@ -1087,10 +1090,6 @@ static int run_steps(dg_handle *h, int max_steps, double fixed_dt, double t_end,
   const bool stops = conv || t_end < HUGE_VAL;
   const double t0 = t_inout ? *t_inout : 0.;
   MeshDev m = mesh_dev(h);
-  if (conv && !h->d_prev && h->cfg.limiter) {
-    int rc = alloc(h, (void **)&h->d_prev, sizeof(double) * dofs(h));
-    if (rc) return rc;
-  }
   int rc = write_state(h, t0, fixed_dt, t_end, conv_tol);
   if (rc) return rc;
   if (h->cfg.limiter) launch_limit(phys, p, m, h->d_c, h->stream);  // time_integrator.cu:179-184
@@ -1099,14 +1098,14 @@ static int run_steps(dg_handle *h, int max_steps, double fixed_dt, double t_end,
     launch_traces(phys, p, h->K, h->d_c, h->d_tr[0], h->stream);
   }
   launch_lambda_init(phys, p, m, h->ph, h->d_c, h->d_st, cfl_mode, h->cfg.cfl * h->min_r,
-                     fixed_dt, t0, 1, nullptr, h->stream, nullptr, 0, h->d_part,
-                     posfix_on(h) && !h->cfg.limiter ? h->d_bad : nullptr);
+                     fixed_dt, t0, 1, nullptr, h->stream, h->d_part,
+                     posfix_on(h) ? h->d_bad : nullptr);
   refresh_bnd_fixed(h, t0);
   HIPCHK(h, hipGetLastError());
   DevState hs;
   std::memset(&hs, 0, sizeof hs);
   // (a small-mesh run leaves its last step to be closed here)
-  const bool fold = !h->cfg.limiter && small_fold(h);
+  const bool fold = small_fold(h);
   auto read_state = [&]() -> int {
     if (fold) {
       FinishArgs f{};
@@ -1125,21 +1124,29 @@ static int run_steps(dg_handle *h, int max_steps, double fixed_dt, double t_end,
   long long launched = 0;
   const long long limit = max_steps < 0 ? (long long)1 << 62 : max_steps;
   HIPCHK(h, hipEventRecord(h->ev0, h->stream));
-  if (h->cfg.limiter) {
-    // limit_c needs every neighbour's finished state: separate launches, one
-    // step at a time when a stop test is active (these launches do not exit on halt)
-    if (!h->d_k[0]) return fail(h, DG_ERR_STATE, "limiter buffers missing");
-    while (launched < limit && !hs.halt && !hs.nan_flag) {
-      limited_step(h, cfl_mode, conv);
-      launched++;
-      if (stops && (rc = read_state())) return rc;
-    }
-    launched *= nstages_of(h->cfg.integrator);
-  } else {
+  {
     StageArgs st[4];
-    const int ns = build_step(h, st, cfl_mode, conv);
+    const int ns = nstages_of(h->cfg.integrator);
+    if (h->cfg.limiter) {
+      if (!h->d_k[0]) return fail(h, DG_ERR_STATE, "limiter buffers missing");
+    } else {
+      build_step(h, st, cfl_mode, conv);
+    }
+    // the launches of n steps from d_c to d_c (limited steps alternate between
+    // d_c and d_b2; an odd number of them ends with a copy)
+    auto record = [&](long long n) {
+      for (long long r = 0; r < n; r++) {
+        if (h->cfg.limiter) {
+          double *b[2] = {h->d_c, h->d_b2};
+          limited_step(h, cfl_mode, conv, b[r & 1], b[(r + 1) & 1]);
+        } else {
+          for (int i = 0; i < ns; i++) launch_stage_bnd(h, st[i]);
+        }
+      }
+      if (h->cfg.limiter && (n & 1)) launch_copy((long long)dofs(h), h->d_c, h->d_b2, h->stream);
+    };
     const bool use_graph = std::getenv("DG_NO_GRAPH") == nullptr;
-    const int key = cfl_mode | (conv ? 2 : 0);
+    const int key = cfl_mode | (conv ? 2 : 0) | (bnd_time_dependent(h) ? 4 : 0);
     if (use_graph && (limit > 1 || stops) && h->graph_key != key) {
       drop_graphs(h);
       // every step launches the same kernels with the same arguments (time,
@@ -1148,8 +1155,7 @@ static int run_steps(dg_handle *h, int max_steps, double fixed_dt, double t_end,
       for (int q = 0; q < kGraphLevels; q++) {
         hipGraph_t g;
         HIPCHK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-        for (int r = 0; r < (1 << q); r++)
-          for (int i = 0; i < ns; i++) launch_stage_bnd(h, st[i]);
+        record(1ll << q);
         HIPCHK(h, hipStreamEndCapture(h->stream, &g));
         hipError_t e = hipGraphInstantiate(&h->graph[q], g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
@@ -1171,8 +1177,8 @@ static int run_steps(dg_handle *h, int max_steps, double fixed_dt, double t_end,
           HIPCHK(h, hipGraphLaunch(h->graph[q], h->stream));
           s += 1ll << q;
         } else {
-          for (int i = 0; i < ns; i++) launch_stage_bnd(h, st[i]);
-          s++;
+          record(chunk);
+          s = chunk;
         }
       }
       steps += chunk;
@@ -1287,7 +1293,7 @@ extern "C" int dg_lambda(dg_handle *h, double *lam) {
   if (!h->K) return fail(h, DG_ERR_STATE, "dg_lambda: no mesh");
   HIPCHK(h, hipSetDevice(h->cfg.device));
   launch_lambda_init(h->cfg.physics, h->cfg.p, mesh_dev(h), h->ph, h->d_c, nullptr, 0, 0., 0., 0.,
-                     0, h->d_lam, h->stream, nullptr, 0, nullptr);
+                     0, h->d_lam, h->stream, nullptr);
   HIPCHK(h, hipGetLastError());
   HIPCHK(h, hipMemcpyAsync(lam, h->d_lam, sizeof(double) * h->K, hipMemcpyDeviceToHost,
                            h->stream));

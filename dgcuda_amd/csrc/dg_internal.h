@@ -129,6 +129,24 @@ struct StageArgs {
 // doubles of stored traces per element: 3 sides x n_q1 points x 4 variables
 __host__ __device__ constexpr int tr_elem(int p) { return 12 * (p + 1); }
 
+// the second launch of a limited stage (k_limited, dg_limit.h)
+struct LimArgs {
+  MeshDev m;
+  PhysParams ph;
+  const double *k;        // dt L(u) of the stage, not limited
+  const double *un, *us;  // step base, stage input
+  double *acc, *out;      // RK4 running combination; next stage's input or the new state
+  const DevState *st;     // the running step's state
+  int mode, accmode;
+  double A, B, C;
+  int final;              // 1: the step's last stage
+  int fix;                // positivity: on the base by its flags, on the output
+  int *bad;               // flags of the base; the last stage writes the new state's
+  int conv;
+  unsigned long long *part;
+  int nblk, small;
+};
+
 // parameters of the step-closing reduction (k_finish)
 struct FinishArgs {
   int cfl_mode;     // 1: dt from the CFL rule
@@ -191,21 +209,16 @@ void launch_exact_vertex(int phys, const MeshDev &m, const PhysParams &ph, doubl
 // step (initial: opens the first) through part and k_finish
 void launch_lambda_init(int phys, int p, const MeshDev &m, const PhysParams &ph, const double *c,
                         DevState *st, int cfl_mode, double cfl_num, double fixed_dt, double t0,
-                        int initial, double *lam_out, hipStream_t s, const double *cprev,
-                        int conv_rows, unsigned long long *part, int *bad_out = nullptr);
+                        int initial, double *lam_out, hipStream_t s, unsigned long long *part,
+                        int *bad_out = nullptr);
 void launch_finish(DevState *st, const unsigned long long *part, int nblk, const FinishArgs &f,
                    hipStream_t s);
 void launch_copy(long long n, double *dst, const double *src, hipStream_t s);
-void launch_posfix(int phys, int p, int K, const PhysParams &ph, double *c, hipStream_t s);
 void launch_flags(int phys, int p, int K, const PhysParams &ph, const double *c, int *bad,
                   hipStream_t s, int *fired = nullptr);
 void launch_limit(int phys, int p, const MeshDev &m, double *c, hipStream_t s);
-void launch_axpy(long long n, double *out, const double *c, double alpha, const double *k,
-                 hipStream_t s);
-void launch_ssp(long long n, double *out, const double *un, double a, const double *us, double b,
-                const double *k, double cc, hipStream_t s);
-void launch_rk4_final(long long n, double *c, const double *k1, const double *k2,
-                      const double *k3, const double *k4, hipStream_t s);
+void launch_limited(int phys, const LimArgs &a, hipStream_t s);
+int limited_blocks(int K, bool small);  // its blocks
 void launch_eval_u(int phys, int p, int K, const double *c, int n, double *u1, double *u2,
                    double *u3, hipStream_t s);
 // boundary data of every boundary slot at the stage time (or a fixed time)

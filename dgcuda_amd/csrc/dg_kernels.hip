@@ -33,6 +33,7 @@
 #include "dg_stage.h"
 #include "dg_stage_q.h"
 #include "dg_stage_s.h"
+#include "dg_limit.h"
 
 namespace dgk {
 
@@ -352,14 +353,13 @@ void launch_exact_vertex(int phys, const MeshDev &m, const PhysParams &ph, doubl
 template <int PHYS, int P>
 __global__ __launch_bounds__(BLK) void k_lambda_init(const MeshDev m, const PhysParams ph,
                                                      const double *c,
-                                                     double *lam_out, const double *cprev,
-                                                     int conv_rows, unsigned long long *part,
+                                                     double *lam_out, unsigned long long *part,
                                                      int *bad_out) {
   constexpr int NP = np_of(P), N = nvars_of(PHYS);
   const Tab<P> &T = tab<P>();
   const int K = m.K;
   const int e = blockIdx.x * BLK + threadIdx.x;
-  double lam = 0., dc = 0.;
+  double lam = 0.;
   if constexpr (has_positivity<PHYS>()) {
     if (bad_out && e < K) {
       double o[N][NP];
@@ -381,22 +381,19 @@ __global__ __launch_bounds__(BLK) void k_lambda_init(const MeshDev m, const Phys
     lam = cfl_speed<PHYS>(pv, U, PHYS == PH_TE ? m.eps[e] : 1.);
     if (lam_out) lam_out[e] = lam;
     lam = ref_max_operand(lam, e);
-    if (cprev)
-      for (int r = 0; r < conv_rows && r < N * NP; r++)
-        dc = fmax(dc, fabs(c[(size_t)r * K + e] - cprev[(size_t)r * K + e]));
   }
-  if (part) block_partials(lam, dc, cprev != nullptr, part, blockIdx.x, gridDim.x);
+  if (part) block_partials(lam, 0., false, part, blockIdx.x, gridDim.x);
 }
 
 void launch_lambda_init(int phys, int p, const MeshDev &m, const PhysParams &ph, const double *c,
                         DevState *st, int cfl_mode, double cfl_num, double fixed_dt, double t0,
-                        int initial, double *lam_out, hipStream_t s, const double *cprev,
-                        int conv_rows, unsigned long long *part, int *bad_out) {
+                        int initial, double *lam_out, hipStream_t s, unsigned long long *part,
+                        int *bad_out) {
   const int nblk = nblocks(m.K, BLK);
   dispatch(phys, p, [&](auto PH, auto PP) {
     constexpr int ph_ = decltype(PH)::value, pp = decltype(PP)::value;
     hipLaunchKernelGGL((k_lambda_init<ph_, pp>), dim3(nblk), dim3(BLK), 0, s, m, ph, c, lam_out,
-                       cprev, conv_rows, st ? part : nullptr, bad_out);
+                       st ? part : nullptr, bad_out);
   });
   if (st) {
     FinishArgs f{};
@@ -406,32 +403,8 @@ void launch_lambda_init(int phys, int p, const MeshDev &m, const PhysParams &ph,
     f.fixed_dt = fixed_dt;
     f.initial = initial;
     f.t0 = t0;
-    f.conv = cprev != nullptr;
     launch_finish(st, part, nblk, f, s);
   }
-}
-
-// element-local positivity fix of a state (race-free check_physical)
-template <int PHYS, int P>
-__global__ __launch_bounds__(BLK) void k_posfix(int K, const PhysParams ph, double *c) {
-  constexpr int NP = np_of(P), N = nvars_of(PHYS);
-  const int e = blockIdx.x * BLK + threadIdx.x;
-  if (e >= K) return;
-  if constexpr (has_positivity<PHYS>()) {
-    double o[N][NP];
-    for (int n = 0; n < N; n++)
-      for (int i = 0; i < NP; i++) o[n][i] = c[(size_t)(n * NP + i) * K + e];
-    if (!elem_physical<PHYS, P>(ph, o))
-      for (int n = 0; n < N; n++)
-        for (int i = 1; i < NP; i++) c[(size_t)(n * NP + i) * K + e] = 0.;
-  }
-}
-
-void launch_posfix(int phys, int p, int K, const PhysParams &ph, double *c, hipStream_t s) {
-  dispatch(phys, p, [&](auto PH, auto PP) {
-    constexpr int ph_ = decltype(PH)::value, pp = decltype(PP)::value;
-    hipLaunchKernelGGL((k_posfix<ph_, pp>), dim3(nblocks(K, BLK)), dim3(BLK), 0, s, K, ph, c);
-  });
 }
 
 // positivity flags of a state (1: it fails the point check, as the stage
@@ -510,43 +483,24 @@ void launch_limit(int phys, int p, const MeshDev &m, double *c, hipStream_t s) {
   });
 }
 
+// Blocks of 16 elements where the stage runs its point-parallel form (the same
+// blocks as its p = 1 ones, so its first stage closes the step from these
+// partials), of 64 elsewhere.
+int limited_blocks(int K, bool small) { return small ? small_blocks(1, K) : nblocks(K, 64); }
+
+void launch_limited(int phys, const LimArgs &a, hipStream_t s) {
+  dispatch(phys, 1, [&](auto PH, auto) {
+    constexpr int ph_ = decltype(PH)::value, n = nvars_of(ph_);
+    if (a.small)
+      hipLaunchKernelGGL((k_limited<ph_, small_eb(1)>), dim3(a.nblk),
+                         dim3(limited_threads(n, small_eb(1))), 0, s, a);
+    else
+      hipLaunchKernelGGL((k_limited<ph_, 64>), dim3(a.nblk), dim3(limited_threads(n, 64)), 0, s,
+                         a);
+  });
+}
+
 // ------------------------------------------------------------ elementwise
-
-__global__ void k_axpy(long long n, double *out, const double *c, double alpha, const double *k) {
-  long long i = (long long)blockIdx.x * BLK + threadIdx.x;
-  if (i < n) out[i] = c[i] + alpha * k[i];  // rk_tempstorage time_integrator.cu:107-113
-}
-
-void launch_axpy(long long n, double *out, const double *c, double alpha, const double *k,
-                 hipStream_t s) {
-  hipLaunchKernelGGL(k_axpy, dim3(nblocks(n, BLK)), dim3(BLK), 0, s, n, out, c, alpha, k);
-}
-
-__global__ void k_ssp(long long n, double *out, const double *un, double a, const double *us,
-                      double b, const double *k, double cc) {
-  long long i = (long long)blockIdx.x * BLK + threadIdx.x;
-  if (i < n) {
-    double v = (a != 0.) ? a * un[i] + b * us[i] : b * us[i];
-    out[i] = v + cc * k[i];
-  }
-}
-
-void launch_ssp(long long n, double *out, const double *un, double a, const double *us, double b,
-                const double *k, double cc, hipStream_t s) {
-  hipLaunchKernelGGL(k_ssp, dim3(nblocks(n, BLK)), dim3(BLK), 0, s, n, out, un, a, us, b, k, cc);
-}
-
-__global__ void k_rk4_final(long long n, double *c, const double *k1, const double *k2,
-                            const double *k3, const double *k4) {
-  long long i = (long long)blockIdx.x * BLK + threadIdx.x;
-  // rk4 time_integrator.cu:124-130
-  if (i < n) c[i] += k1[i] / 6. + k2[i] / 3. + k3[i] / 3. + k4[i] / 6.;
-}
-
-void launch_rk4_final(long long n, double *c, const double *k1, const double *k2,
-                      const double *k3, const double *k4, hipStream_t s) {
-  hipLaunchKernelGGL(k_rk4_final, dim3(nblocks(n, BLK)), dim3(BLK), 0, s, n, c, k1, k2, k3, k4);
-}
 
 __global__ void k_copy(long long n, double *dst, const double *src) {
   long long i = (long long)blockIdx.x * BLK + threadIdx.x;

@@ -137,3 +137,39 @@ def test_stops_and_time_dependent_boundaries_on_a_small_mesh():
         assert rel_l2(s.coeffs(), o.coeffs()) < TOL
         assert "conv_tol" not in kw or abs(c - co) <= 1e-12 * abs(co)
     s.close()
+
+
+@pytest.mark.parametrize("physics,integrator,K", [
+    (L.EULER, L.RK4, 18), (L.EULER, L.RK4, 12168), (L.EULER, L.RK4, 12482),
+    (L.EULER, L.SSPRK3, 2178), (L.EULER, L.SSPRK3, 20000),
+    (L.EULER, L.RK2MID, 578), (L.SWE, L.SSPRK2, 1058), (L.SWE, L.SSPRK3, 18050),
+    (L.MAXWELL_TE, L.RK4, 338), (L.ADVECTION, L.RK4, 392),
+    (L.ADVECTION, L.SSPRK2, 15138)])
+def test_limited_steps_either_side_of_the_size_rule(physics, integrator, K):
+    """the limiter's second launch (16 or 64 elements per block) against the
+    oracle: odd and even runs (the state's two buffers), then a stop at t_end
+    inside a chunk of steps and one on the step-to-step change"""
+    s, o = _pair(physics, 1, K, periodic=False, integrator=integrator, cfl=0.2, limiter=True)
+    u = o.coeffs()
+    u = u * (1.0 + 0.05 * np.random.default_rng(K).standard_normal(u.shape))
+    if physics in (L.EULER, L.SWE):
+        u[:, 1:, ::41] *= 40.0  # elements that contribute their means only
+    s.set_coeffs(u)
+    o.set_coeffs(u)
+    print("limited physics", physics, "K", s.K, "integrator", integrator, flush=True)
+    t = to = 0.0
+    for n in (1, 2, 5):
+        t, dt = s.step(n, t=t)
+        rc, to, _, _, dto = o.run_until(max_steps=n, t0=to)
+        r = rel_l2(s.coeffs(), o.coeffs())
+        print("  steps", n, "rel", r, "t", t, to)
+        assert rc == 0 and abs(t - to) <= 1e-13 * to and abs(dt - dto) <= 1e-13 * dto
+        assert r < TOL
+    for kw in (dict(t_end=t + 2.5 * dt), dict(max_steps=4, conv_tol=0.0)):
+        t, n, c = s.run(t=t, **kw)
+        rc, to, no, co, _ = o.run_until(t0=to, **kw)
+        r = rel_l2(s.coeffs(), o.coeffs())
+        print("  stop", kw, n, no, "rel", r, "change", c, co)
+        assert rc == 0 and n == no and abs(t - to) <= 1e-13 * to and r < TOL
+        assert "conv_tol" not in kw or abs(c - co) <= 1e-10 * abs(co)
+    s.close()
