@@ -56,6 +56,7 @@ struct dg_handle {
   std::vector<double> hV;
   std::vector<int> h_bnd_elem, h_bnd_code, h_bnd_side;
   bool user_bnd = false;  // the caller's boundary states replace the problem's
+  bool bnd_ready = false;  // d_bnd_val holds the problem's, which do not depend on time
   bool use_traces = true;  // runs of steps may store traces (traces_wanted)
   // state: d_c, d_b1, d_b2 (and d_acc) are views into one allocation,
   // d_state (block_views)
@@ -69,6 +70,10 @@ struct dg_handle {
   double *d_err = nullptr, *d_lam = nullptr;
   DevState *d_st = nullptr;  // [2]: the state between steps, the running step's (k_stage_s)
   unsigned long long *d_part = nullptr;  // per-block maxima of the step reduction
+  char *d_ws = nullptr;                  // dg_adjoint_solve's buffers, kept for the next call
+  size_t ws_bytes = 0;
+  double *d_red = nullptr;               // [kSumBlocks + 1] objective sum: partials, result
+  double *d_gu = nullptr;                // dg_adjoint_rhs's output before its copy out
   int *d_bad = nullptr;                  // positivity flags of the stored state d_c
   // graphs of 2^q steps, q < kGraphLevels (same configuration key)
   hipGraphExec_t graph[kGraphLevels] = {};
@@ -114,6 +119,13 @@ static int alloc(dg_handle *h, void **p, size_t bytes) {
     *p = nullptr;
   }
   hipError_t e = hipMalloc(p, bytes ? bytes : 8);
+  if (e != hipSuccess && h->d_ws && *p != h->d_ws) {  // the kept adjoint buffers go first
+    (void)hipGetLastError();
+    (void)hipFree(h->d_ws);
+    h->d_ws = nullptr;
+    h->ws_bytes = 0;
+    e = hipMalloc(p, bytes ? bytes : 8);
+  }
   if (e != hipSuccess)
     return fail(h, DG_ERR_HIP, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
   return DG_OK;
@@ -351,13 +363,15 @@ static void free_mesh(dg_handle *h) {
   dfree(h->d_bnd_elem); dfree(h->d_bnd_code); dfree(h->d_bnd_val); dfree(h->d_side);
   h->nb_bnd = 0;
   h->bnd_dirichlet = false;
-  h->user_bnd = false;
+  h->user_bnd = h->bnd_ready = false;
   dfree(h->d_state);
   h->d_c = h->d_b1 = h->d_b2 = h->d_acc = nullptr;
   dfree(h->d_trblk);
   for (auto &t : h->d_tr) t = nullptr;
   for (auto &k : h->d_k) dfree(k);
-  dfree(h->d_err); dfree(h->d_lam); dfree(h->d_gw); dfree(h->d_part); dfree(h->d_bad);
+  dfree(h->d_err); dfree(h->d_lam); dfree(h->d_gw); dfree(h->d_gu);
+  dfree(h->d_ws); dfree(h->d_red);
+  h->ws_bytes = 0; dfree(h->d_part); dfree(h->d_bad);
   drop_graphs(h);
   // no mesh from here until a new one is fully uploaded: every call that
   // needs one checks K, and the objective's weights went with the buffers
@@ -735,9 +749,17 @@ static bool bnd_time_dependent(const dg_handle *h) {
           h->cfg.problem == DG_PROB_ADV_ROTHILL);
 }
 
-// boundary data at a fixed time (once per call when it does not change)
+// whether d_bnd_val has to be formed for time t: not the caller's states, and
+// walls and fixed states once per mesh (the caller launches what forms it)
+static bool bnd_stale(dg_handle *h) {
+  if (!h->nb_bnd || h->user_bnd || h->bnd_ready) return false;
+  h->bnd_ready = !bnd_time_dependent(h);
+  return true;
+}
+
+// boundary data at a fixed time
 static void refresh_bnd_fixed(dg_handle *h, double t) {
-  if (h->nb_bnd && !h->user_bnd)
+  if (bnd_stale(h))
     launch_bnd(h->cfg.physics, h->cfg.p, mesh_dev(h), h->ph, h->d_st, 0., 0, t, h->stream);
 }
 
@@ -751,31 +773,61 @@ static void launch_stage_bnd(dg_handle *h, const StageArgs &a) {
   launch_stage(h->cfg.physics, h->cfg.p, s, h->stream);
 }
 
+// Whether a kernel on the handle's device can use the caller's array p in
+// place: a DG_DEVICE array in plain memory of that very device (a copy also
+// takes another device's or managed memory), aligned for doubles.
+static bool in_place(const dg_handle *h, const void *p, int where) {
+  if (where != DG_DEVICE || ((uintptr_t)p & 7)) return false;
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return at.type == hipMemoryTypeDevice && !at.isManaged && at.device == h->cfg.device;
+}
+
+static bool overlap(const void *a, const void *b, size_t bytes) {
+  return (const char *)a < (const char *)b + bytes && (const char *)b < (const char *)a + bytes;
+}
+
+// k = dt L(u) into out: one launch before the stage (k_prep)
+static void rhs_launches(dg_handle *h, const double *u, double t, double dt, double *out,
+                         DevState *st, int *bad, bool bnd) {
+  StageArgs a = base_args(h);
+  a.st = st;
+  a.bad = bad;
+  a.us = u;
+  a.un = u;
+  a.out = out;
+  a.mode = M_KONLY;
+  // the positivity prepass on the input, through its flags (the stage
+  // kernel takes a neighbour's fix from its flag)
+  a.fix_in = a.flags_in = posfix_on(h) ? 1 : 0;
+  launch_prep(h->cfg.physics, h->cfg.p, a.m, h->ph, a.fix_in ? u : nullptr, bad, st, t, dt,
+              bnd, h->stream);
+  launch_stage(h->cfg.physics, h->cfg.p, a, h->stream);
+}
+
+// Device arrays are read and written in place (Euler p = 1 on 1,080 triangles:
+// 25.9 us a call; 32.7 with the input, the output and the step state copied and
+// the flags launched by themselves).  The stage gathers neighbours of u while
+// it stores k, so overlapping arrays, as host data, go through the handle's
+// buffers.
 extern "C" int dg_eval_rhs(dg_handle *h, const double *u, double t, double dt, double *k,
                            int where) {
   if (!h || !u || !k) return DG_ERR_ARG;
   if (!h->K) return fail(h, DG_ERR_STATE, "dg_eval_rhs: no mesh");
   HIPCHK(h, hipSetDevice(h->cfg.device));
   const size_t sb = sizeof(double) * dofs(h);
-  HIPCHK(h, hipMemcpyAsync(h->d_b1, u, sb, kind_to(where), h->stream));
-  int rc = write_state(h, t, dt);
-  if (rc) return rc;
-  StageArgs a = base_args(h);
-  a.us = h->d_b1;
-  a.un = h->d_b1;
-  a.out = h->d_b2;
-  a.mode = M_KONLY;
-  if (posfix_on(h)) {
-    // the positivity prepass on the input, through its flags (the stage
-    // kernel takes a neighbour's fix from its flag)
-    launch_flags(h->cfg.physics, h->cfg.p, h->K, h->ph, h->d_b1, h->d_bad, h->stream);
-    a.fix_in = 1;
-    a.flags_in = 1;
+  if (in_place(h, u, where) && in_place(h, k, where) && !overlap(u, k, sb)) {
+    rhs_launches(h, u, t, dt, k, h->d_st, h->d_bad, bnd_stale(h));
+    HIPCHK(h, hipGetLastError());
+  } else {
+    HIPCHK(h, hipMemcpyAsync(h->d_b1, u, sb, kind_to(where), h->stream));
+    rhs_launches(h, h->d_b1, t, dt, h->d_b2, h->d_st, h->d_bad, bnd_stale(h));
+    HIPCHK(h, hipGetLastError());
+    HIPCHK(h, hipMemcpyAsync(k, h->d_b2, sb, kind_from(where), h->stream));
   }
-  refresh_bnd_fixed(h, t);
-  launch_stage(h->cfg.physics, h->cfg.p, a, h->stream);
-  HIPCHK(h, hipGetLastError());
-  HIPCHK(h, hipMemcpyAsync(k, h->d_b2, sb, kind_from(where), h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
   return DG_OK;
 }
@@ -822,7 +874,7 @@ extern "C" int dg_set_boundary_states(dg_handle *h, const double *U, int where) 
   if (!h) return DG_ERR_ARG;
   if (!h->K) return fail(h, DG_ERR_STATE, "dg_set_boundary_states: no mesh");
   HIPCHK(h, hipSetDevice(h->cfg.device));
-  h->user_bnd = false;
+  h->user_bnd = h->bnd_ready = false;
   if (!U || !h->nb_bnd) return DG_OK;  // the problem's boundary data again
   const size_t NQ1 = h->nq1, N = h->N, nb = h->nb_bnd;
   std::vector<double> u(nb * NQ1 * N), bv(nb * NQ1 * NMAX, 0.);
@@ -866,30 +918,14 @@ extern "C" int dg_eval_rhs_noalloc(dg_handle *h, const double *u, double t, doub
                 "dg_eval_rhs_noalloc: K = %d elements exceed the fixed scratch's %d", h->K,
                 kScratchMaxK);
   const size_t sb = sizeof(double) * dofs(h);
-  const char *ub = (const char *)u, *kb = (const char *)k;
-  if (ub < kb + sb && kb < ub + sb)
+  if (overlap(u, k, sb))
     return fail(h, DG_ERR_ARG, "dg_eval_rhs_noalloc: u and k overlap (k is written while u is read)");
   const int dev = h->cfg.device;
   char *scr = (char *)g_scratch[dev];
   if (!scr) return fail(h, DG_ERR_STATE, "dg_eval_rhs_noalloc: no scratch address for device %d", dev);
   HIPCHK(h, hipSetDevice(dev));
-  DevState *st = (DevState *)scr;
-  int *bad = (int *)(scr + 256);
-  launch_set_state(st, t, dt, h->stream);
-  StageArgs a = base_args(h);
-  a.st = st;
-  a.bad = bad;
-  a.us = u;
-  a.un = u;
-  a.out = k;
-  a.mode = M_KONLY;
-  if (posfix_on(h)) {
-    launch_flags(h->cfg.physics, h->cfg.p, h->K, h->ph, u, bad, h->stream);
-    a.fix_in = 1;
-    a.flags_in = 1;
-  }
-  refresh_bnd_fixed(h, t);
-  launch_stage(h->cfg.physics, h->cfg.p, a, h->stream);
+  // (a captured call forms the boundary data whenever it is replayed)
+  rhs_launches(h, u, t, dt, k, (DevState *)scr, (int *)(scr + 256), h->nb_bnd && !h->user_bnd);
   HIPCHK(h, hipGetLastError());
   return DG_OK;
 }
@@ -1147,39 +1183,46 @@ static int run_steps(dg_handle *h, int max_steps, double fixed_dt, double t_end,
     };
     const bool use_graph = std::getenv("DG_NO_GRAPH") == nullptr;
     const int key = cfl_mode | (conv ? 2 : 0) | (bnd_time_dependent(h) ? 4 : 0);
-    if (use_graph && (limit > 1 || stops) && h->graph_key != key) {
+    // Every step launches the same kernels with the same arguments (time, dt
+    // and the stop state live on the device), so a run of steps is the one-step
+    // sequence repeated.  A level is captured by the first run that uses it:
+    // all six are 63 steps, most of a first short run's time.
+    const bool capture = use_graph && (limit > 1 || stops);
+    if (capture && h->graph_key != key) {
       drop_graphs(h);
-      // every step launches the same kernels with the same arguments (time,
-      // dt and the stop state live on the device), so a run of steps is the
-      // one-step sequence repeated
-      for (int q = 0; q < kGraphLevels; q++) {
-        hipGraph_t g;
-        HIPCHK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-        record(1ll << q);
-        HIPCHK(h, hipStreamEndCapture(h->stream, &g));
-        hipError_t e = hipGraphInstantiate(&h->graph[q], g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (e != hipSuccess) return fail(h, DG_ERR_HIP, "graph instantiate: %s", hipGetErrorString(e));
-        HIPCHK(h, hipGraphUpload(h->graph[q], h->stream));
-      }
       h->graph_key = key;
     }
     const bool graph = use_graph && h->graph_key == key;
+    auto level = [&](int q) -> int {
+      if (h->graph[q] || !capture) return DG_OK;
+      hipGraph_t g;
+      HIPCHK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
+      record(1ll << q);
+      HIPCHK(h, hipStreamEndCapture(h->stream, &g));
+      hipError_t e = hipGraphInstantiate(&h->graph[q], g, nullptr, nullptr, 0);
+      (void)hipGraphDestroy(g);
+      if (e != hipSuccess) {
+        h->graph[q] = nullptr;
+        return fail(h, DG_ERR_HIP, "graph instantiate: %s", hipGetErrorString(e));
+      }
+      HIPCHK(h, hipGraphUpload(h->graph[q], h->stream));
+      return DG_OK;
+    };
     long long steps = 0;
     while (steps < limit && !hs.halt && !hs.nan_flag) {
       // launches after a stop exit at once; chunks bound the wasted launches
       const long long chunk = stops ? std::min<long long>(limit - steps, 32) : limit - steps;
       for (long long s = 0; s < chunk;) {
-        if (graph) {
-          // the largest graph that fits the steps left
-          int q = kGraphLevels - 1;
-          while ((1ll << q) > chunk - s) q--;
+        // the largest graph that fits the steps left
+        int q = kGraphLevels - 1;
+        while ((1ll << q) > chunk - s) q--;
+        if ((rc = level(q)) != DG_OK) return rc;
+        if (graph && h->graph[q]) {
           HIPCHK(h, hipGraphLaunch(h->graph[q], h->stream));
-          s += 1ll << q;
         } else {
-          record(chunk);
-          s = chunk;
+          record(1ll << q);
         }
+        s += 1ll << q;
       }
       steps += chunk;
       if (stops && (rc = read_state())) return rc;
@@ -1407,35 +1450,80 @@ Butcher butcher_of(int integ) {
 }  // namespace
 
 
-// Device buffers of the adjoint: each adj_alloc call makes one allocation
-// and hands out its buffers at 256-byte-aligned offsets, each 8 KiB past a
-// 256-byte multiple of the one before (one hipMalloc per group rather than
-// per buffer: a sweep may hold thousands of buffers).  With the 8 KiB pad the
-// config-5 sweep ran 1.8 % faster than without (2, 4 and 16 KiB: 1.3-1.5 %);
-// the forward's state buffers (block_views) measured no gain from a pad.
+// Device buffers of the adjoint: a group's buffers lie at 256-byte-aligned
+// offsets, each 8 KiB past a 256-byte multiple of the one before.  With the
+// 8 KiB pad the config-5 sweep ran 1.8 % faster than without (2, 4 and 16 KiB:
+// 1.3-1.5 %); the forward's state buffers (block_views) measured no gain from
+// a pad.
 struct AdjBuffers {
   std::vector<double *> bufs;
-  std::vector<void *> blocks;
+  void *block = nullptr;  // the group's own allocation, if it has one
   AdjBuffers() = default;
   AdjBuffers(const AdjBuffers &) = delete;
   AdjBuffers &operator=(const AdjBuffers &) = delete;
   ~AdjBuffers() {
-    for (void *p : blocks) (void)hipFree(p);
+    if (block) (void)hipFree(block);
   }
 };
 
+static size_t adj_stride(size_t bytes) { return (bytes + 255) / 256 * 256 + 8192; }
+
+static void adj_views(AdjBuffers &ab, char *base, size_t count, size_t bytes) {
+  for (size_t q = 0; q < count; q++) ab.bufs.push_back((double *)(base + q * adj_stride(bytes)));
+}
+
+// a group with an allocation of its own
 static int adj_alloc(dg_handle *h, AdjBuffers &ab, size_t count, size_t bytes) {
   if (!count) return DG_OK;
-  const size_t stride = (bytes + 255) / 256 * 256 + 8192;
   void *p = nullptr;
-  hipError_t e = hipMalloc(&p, stride * count);
+  hipError_t e = hipMalloc(&p, adj_stride(bytes) * count);
   if (e != hipSuccess)
     return fail(h, DG_ERR_HIP, "adjoint: hipMalloc of %zu buffers of %zu bytes failed (%s)", count,
                 bytes, hipGetErrorString(e));
-  ab.blocks.push_back(p);
-  for (size_t q = 0; q < count; q++) ab.bufs.push_back((double *)((char *)p + q * stride));
+  ab.block = p;
+  adj_views(ab, (char *)p, count, bytes);
   return DG_OK;
 }
+
+// The work buffers of a solve lie in one allocation that the handle keeps for
+// the next solve, up to 1/32 of the device's memory (9 GB): allocating and
+// freeing them was 1.7 ms of a 33 ms gradient (TE p = 3, 199,712 triangles, 32
+// steps, 5.6 GB) and 1.0 of 10.4 (Euler p = 4, 131,072, 8 steps).  Larger ones
+// are given back at once; the rest with the mesh, or when an allocation fails.
+struct AdjWorkspace {
+  dg_handle *h;
+  char *p = nullptr;
+  size_t used = 0;
+  explicit AdjWorkspace(dg_handle *hh) : h(hh) {}
+  AdjWorkspace(const AdjWorkspace &) = delete;
+  ~AdjWorkspace() {
+    if (!h->d_ws) return;
+    size_t fr = 0, tot = 0;
+    if (hipMemGetInfo(&fr, &tot) != hipSuccess) (void)hipGetLastError();
+    if (h->ws_bytes <= tot / 32) return;
+    dfree(h->d_ws);
+    h->ws_bytes = 0;
+  }
+  int reserve(size_t bytes) {
+    if (h->ws_bytes < bytes) {
+      dfree(h->d_ws);
+      h->ws_bytes = 0;
+      const hipError_t e = hipMalloc((void **)&h->d_ws, bytes);
+      if (e != hipSuccess) {
+        h->d_ws = nullptr;
+        return fail(h, DG_ERR_HIP, "adjoint: hipMalloc of %zu bytes failed (%s)", bytes,
+                    hipGetErrorString(e));
+      }
+      h->ws_bytes = bytes;
+    }
+    p = h->d_ws;
+    return DG_OK;
+  }
+  void take(AdjBuffers &ab, size_t count, size_t bytes) {
+    adj_views(ab, p + used, count, bytes);
+    used += adj_stride(bytes) * count;
+  }
+};
 
 // How many of a checkpointed solve's segments keep the stage data of the
 // forward pass itself (the last ones), so that the reverse sweep walks them
@@ -1505,34 +1593,27 @@ extern "C" int dg_adjoint_set_objective(dg_handle *h, int kind, const double *pa
 
 static bool adjoint_supported(const dg_handle *h) { return !h->cfg.limiter; }
 
-// objective value of d_c and its gradient into gout (device)
+// objective value of d_c and its gradient into gout (device; nullptr: none)
 static int eval_objective(dg_handle *h, double *J, double *gout) {
   const size_t n = dofs(h);
-  if (h->obj_kind == DG_OBJ_LINEAR) {
-    std::vector<double> c(n), g(n);
-    HIPCHK(h, hipMemcpyAsync(c.data(), h->d_c, sizeof(double) * n, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(g.data(), h->d_gw, sizeof(double) * n, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(gout, h->d_gw, sizeof(double) * n, hipMemcpyDeviceToDevice, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    double s = 0.;
-    for (size_t i = 0; i < n; i++) s += g[i] * c[i];
-    *J = s;
-    return DG_OK;
+  if (!h->d_red) {
+    const int rc = alloc(h, (void **)&h->d_red, sizeof(double) * (kSumBlocks + 1));
+    if (rc) return rc;
   }
-  double *prm = nullptr;
-  HIPCHK(h, hipMalloc((void **)&prm, 8 * sizeof(double)));
-  HIPCHK(h, hipMemcpyAsync(prm, h->obj_params.data(), 8 * sizeof(double), hipMemcpyHostToDevice,
-                           h->stream));
-  launch_objective(h->cfg.physics, h->cfg.p, h->obj_kind, mesh_dev(h), h->ph, h->d_c, prm,
-                   h->d_lam, gout, h->stream);
-  std::vector<double> v(h->K);
-  HIPCHK(h, hipMemcpyAsync(v.data(), h->d_lam, sizeof(double) * h->K, hipMemcpyDeviceToHost,
+  if (h->obj_kind == DG_OBJ_LINEAR) {
+    if (gout) launch_copy((long long)n, gout, h->d_gw, h->stream);
+    launch_sum((long long)n, h->d_gw, h->d_c, h->d_red, h->stream);
+  } else {
+    ObjParams prm;
+    std::copy_n(h->obj_params.begin(), 8, prm.v);
+    launch_objective(h->cfg.physics, h->cfg.p, h->obj_kind, mesh_dev(h), h->ph, h->d_c, prm,
+                     h->d_lam, gout, h->stream);
+    launch_sum(h->K, h->d_lam, nullptr, h->d_red, h->stream);
+  }
+  HIPCHK(h, hipGetLastError());
+  HIPCHK(h, hipMemcpyAsync(J, h->d_red + kSumBlocks, sizeof(double), hipMemcpyDeviceToHost,
                            h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  (void)hipFree(prm);
-  double s = 0.;
-  for (int e = 0; e < h->K; e++) s += v[e];
-  *J = s;
   return DG_OK;
 }
 
@@ -1562,16 +1643,27 @@ extern "C" int dg_adjoint_rhs(dg_handle *h, const double *u, double t, double dt
                 "adjoint: the limiter is not differentiated");
   HIPCHK(h, hipSetDevice(h->cfg.device));
   const size_t sb = sizeof(double) * dofs(h);
-  AdjBuffers ab;
-  int rc = adj_alloc(h, ab, 1, sb);
-  if (rc) return rc;
-  HIPCHK(h, hipMemcpyAsync(h->d_b1, u, sb, kind_to(where), h->stream));
-  HIPCHK(h, hipMemcpyAsync(h->d_b2, gk, sb, kind_to(where), h->stream));
+  // in place as dg_eval_rhs, else through the handle's buffers (the output's
+  // is made by the first such call and goes with the mesh)
+  const bool direct = in_place(h, u, where) && in_place(h, gk, where) && in_place(h, gu, where) &&
+                      !overlap(u, gu, sb) && !overlap(gk, gu, sb);
+  const double *ui = u, *gi = gk;
+  double *go = gu;
+  if (!direct) {
+    if (!h->d_gu) {
+      const int rc = alloc(h, (void **)&h->d_gu, sb);
+      if (rc) return rc;
+    }
+    HIPCHK(h, hipMemcpyAsync(h->d_b1, u, sb, kind_to(where), h->stream));
+    HIPCHK(h, hipMemcpyAsync(h->d_b2, gk, sb, kind_to(where), h->stream));
+    ui = h->d_b1;
+    gi = h->d_b2;
+    go = h->d_gu;
+  }
   refresh_bnd_fixed(h, t);
-  launch_adjoint_rhs(h->cfg.physics, h->cfg.p, adj_args(h, h->d_b1, h->d_b2, ab.bufs[0], nullptr, dt),
-                     h->stream);
+  launch_adjoint_rhs(h->cfg.physics, h->cfg.p, adj_args(h, ui, gi, go, nullptr, dt), h->stream);
   HIPCHK(h, hipGetLastError());
-  HIPCHK(h, hipMemcpyAsync(gu, ab.bufs[0], sb, kind_from(where), h->stream));
+  if (!direct) HIPCHK(h, hipMemcpyAsync(gu, go, sb, kind_from(where), h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
   return DG_OK;
 }
@@ -1599,19 +1691,26 @@ extern "C" int dg_adjoint_solve(dg_handle *h, int nsteps, double dt, int every, 
   const bool want_eps = te && grad_eps;
   const size_t kst_b = sizeof(double) * 2 * h->np * h->K;
   AdjBuffers ck, store, kst, wk;
-  int rc = adj_alloc(h, wk, S + 3, sb);
-  if (rc) return rc;
+  int rc;
   if (traces_wanted(h) && (rc = alloc_traces(h)) != DG_OK) return rc;
   const int nres = resident_segments(nsteps, every, nseg, sb, [&](int ns) {
     return ((size_t)ns * S + 1) * sb + (want_eps ? (size_t)ns * S * kst_b : 0);
   });
   const int nrec = nseg - nres;  // segments 0 .. nrec - 1 are recomputed
   h->adj_resident = nres;
+  const size_t seg_stages = nrec > 0 ? (size_t)every * S : 0;
+  size_t need = adj_stride(sb) * (S + 3);
+  if (nrec > 0) need += adj_stride(sb) * (nrec + seg_stages + 1);
+  if (want_eps)
+    need += adj_stride(kst_b) * seg_stages + adj_stride(sizeof(double) * h->K) +
+            adj_stride(2 * sizeof(double) * h->S);
+  AdjWorkspace ws(h);
+  if ((rc = ws.reserve(need)) != DG_OK) return rc;
+  ws.take(wk, S + 3, sb);
   if (nrec > 0) {
-    rc = adj_alloc(h, ck, nrec, sb);
-    if (!rc) rc = adj_alloc(h, store, (size_t)every * S + 1, sb);
-    if (!rc && want_eps) rc = adj_alloc(h, kst, (size_t)every * S, kst_b);
-    if (rc) return rc;
+    ws.take(ck, nrec, sb);
+    ws.take(store, seg_stages + 1, sb);
+    if (want_eps) ws.take(kst, seg_stages, kst_b);
   }
   std::vector<AdjBuffers> rstore(nres), rkst(nres);
   for (int j = 0; j < nres; j++) {
@@ -1620,19 +1719,13 @@ extern "C" int dg_adjoint_solve(dg_handle *h, int nsteps, double dt, int every, 
     if (!rc && want_eps) rc = adj_alloc(h, rkst[j], (size_t)ns * S, kst_b);
     if (rc) return rc;
   }
-  // (each buffer's owner is set before the next call that can return early)
-  struct Free {
-    double *p;
-    ~Free() {
-      if (p) (void)hipFree(p);
-    }
-  } fgeps{nullptr}, fgzs{nullptr};
   double *d_geps = nullptr, *d_gzs = nullptr;
   if (want_eps) {
-    HIPCHK(h, hipMalloc((void **)&d_geps, sizeof(double) * h->K));
-    fgeps.p = d_geps;
-    HIPCHK(h, hipMalloc((void **)&d_gzs, 2 * sizeof(double) * h->S));
-    fgzs.p = d_gzs;
+    AdjBuffers g, z;
+    ws.take(g, 1, sizeof(double) * h->K);
+    ws.take(z, 1, 2 * sizeof(double) * h->S);
+    d_geps = g.bufs[0];
+    d_gzs = z.bufs[0];
     HIPCHK(h, hipMemsetAsync(d_geps, 0, sizeof(double) * h->K, h->stream));
   }
   double *G = wk.bufs[S];
@@ -1882,10 +1975,7 @@ extern "C" int dg_adjoint_objective(dg_handle *h, double *J) {
   if (!h->K) return fail(h, DG_ERR_STATE, "dg_adjoint_objective: no mesh");
   if (h->obj_kind < 0) return fail(h, DG_ERR_STATE, "dg_adjoint_objective: no objective set");
   HIPCHK(h, hipSetDevice(h->cfg.device));
-  AdjBuffers ab;
-  int rc = adj_alloc(h, ab, 1, sizeof(double) * dofs(h));
-  if (rc) return rc;
-  return eval_objective(h, J, ab.bufs[0]);
+  return eval_objective(h, J, nullptr);
 }
 
 extern "C" int dg_adjoint_timing(dg_handle *h, double *fwd_ms, double *rev_ms) {

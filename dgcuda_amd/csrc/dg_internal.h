@@ -192,7 +192,6 @@ int ens_vgprs(int phys, int B);
 // byte 0, the positivity flags ([K] ints, K <= kScratchMaxK) at byte 256
 constexpr int kScratchMaxK = 1 << 22;
 int scratch_address(void **p);
-void launch_set_state(DevState *st, double t, double dt, hipStream_t s);
 
 // launchers (dg_kernels.hip)
 int upload_tables(int p, const void *tab, size_t bytes);
@@ -216,6 +215,8 @@ void launch_finish(DevState *st, const unsigned long long *part, int nblk, const
 void launch_copy(long long n, double *dst, const double *src, hipStream_t s);
 void launch_flags(int phys, int p, int K, const PhysParams &ph, const double *c, int *bad,
                   hipStream_t s, int *fired = nullptr);
+void launch_prep(int phys, int p, const MeshDev &m, const PhysParams &ph, const double *u, int *bad,
+                 DevState *st, double t, double dt, bool bnd, hipStream_t s);
 void launch_limit(int phys, int p, const MeshDev &m, double *c, hipStream_t s);
 void launch_limited(int phys, const LimArgs &a, hipStream_t s);
 int limited_blocks(int K, bool small);  // its blocks
@@ -256,8 +257,14 @@ struct AdjArgs {
   double scale;
 };
 void launch_adjoint_rhs(int phys, int p, const AdjArgs &a, hipStream_t s);
+struct ObjParams {
+  double v[8];
+};
 void launch_objective(int phys, int p, int kind, const MeshDev &m, const PhysParams &ph,
-                      const double *c, const double *prm, double *obj_elem, double *grad,
+                      const double *c, const ObjParams &prm, double *obj_elem, double *grad,
                       hipStream_t s);
+// red[kSumBlocks] = sum_i a_i (b: a_i b_i); red [kSumBlocks + 1]
+constexpr int kSumBlocks = 256;
+void launch_sum(long long n, const double *a, const double *b, double *red, hipStream_t s);
 
 }  // namespace dgk

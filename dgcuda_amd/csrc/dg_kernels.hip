@@ -23,6 +23,7 @@
 // per wavefront.  Element blocks are remapped so that each of the 8 XCDs
 // gets a contiguous range of elements (neighbour gathers then hit the XCD's
 // own L2).
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -83,23 +84,6 @@ int scratch_address(void **p) {
   *p = nullptr;
   const hipError_t e = hipGetSymbolAddress(p, HIP_SYMBOL(scratch));
   return e == hipSuccess && *p ? 0 : -1;
-}
-
-// the stage state of a single right-hand-side evaluation at (t, dt), written
-// by a kernel (no memset or copy: the launch sequence stays capturable)
-__global__ void k_set_state(DevState *st, double t, double dt) {
-  DevState s;
-  __builtin_memset(&s, 0, sizeof s);
-  s.t = t;
-  s.dt = dt;
-  s.tdone = t;
-  s.t_end = __builtin_huge_val();
-  s.conv_tol = -1.;
-  *st = s;
-}
-
-void launch_set_state(DevState *st, double t, double dt, hipStream_t s) {
-  hipLaunchKernelGGL(k_set_state, dim3(1), dim3(1), 0, s, st, t, dt);
 }
 
 __global__ __launch_bounds__(BLK) void k_finish(DevState *st, const unsigned long long *part,
@@ -432,6 +416,48 @@ void launch_flags(int phys, int p, int K, const PhysParams &ph, const double *c,
     constexpr int ph_ = decltype(PH)::value, pp = decltype(PP)::value;
     hipLaunchKernelGGL((k_flags<ph_, pp>), dim3(nblocks(K, BLK)), dim3(BLK), 0, s, K, ph, c, bad,
                        fired);
+  });
+}
+
+// What one right-hand-side evaluation at (t, dt) needs before its stage, in
+// one launch: the step state (written by a kernel, with no memset or copy, so
+// the sequence stays capturable), the positivity flags of its input u
+// (nullptr: none) and, with bnd, the boundary data at t.  On 1,080 triangles
+// the three launches and the copy of the state that this replaces were most
+// of the call.
+template <int PHYS, int P>
+__global__ __launch_bounds__(BLK) void k_prep(const MeshDev m, const PhysParams ph,
+                                              const double *u, int *bad, DevState *st, double t,
+                                              double dt, int bnd) {
+  constexpr int NP = np_of(P), N = nvars_of(PHYS);
+  const int e = blockIdx.x * BLK + threadIdx.x, K = m.K;
+  if (e == 0) {
+    DevState s;
+    __builtin_memset(&s, 0, sizeof s);
+    s.t = t;
+    s.dt = dt;
+    s.tdone = t;
+    s.t_end = __builtin_huge_val();
+    s.conv_tol = -1.;
+    *st = s;
+  }
+  if constexpr (has_positivity<PHYS>()) {
+    if (u && e < K) {
+      double o[N][NP];
+      load_state(u, K, e, o);
+      bad[e] = needs_fix<PHYS, P>(ph, o) ? 1 : 0;
+    }
+  }
+  if (bnd && e < m.nb_bnd) bnd_slot<PHYS, P>(m, ph, t, e);
+}
+
+void launch_prep(int phys, int p, const MeshDev &m, const PhysParams &ph, const double *u, int *bad,
+                 DevState *st, double t, double dt, bool bnd, hipStream_t s) {
+  const int n = std::max(u ? m.K : 1, bnd ? m.nb_bnd : 1);
+  dispatch(phys, p, [&](auto PH, auto PP) {
+    constexpr int ph_ = decltype(PH)::value, pp = decltype(PP)::value;
+    hipLaunchKernelGGL((k_prep<ph_, pp>), dim3(nblocks(n, BLK)), dim3(BLK), 0, s, m, ph, u, bad,
+                       st, t, dt, bnd ? 1 : 0);
   });
 }
 

@@ -71,6 +71,7 @@ class Solver:
             if x.device.type == "cuda":
                 self._check_device(x, name)
                 x = x.contiguous()
+                self._wait(x)
                 return x.data_ptr(), _lib.DEVICE, x
             x = x.detach().contiguous().numpy()
         a = np.ascontiguousarray(x, np.float64)
@@ -96,6 +97,13 @@ class Solver:
                 not out.flags["C_CONTIGUOUS"] or out.size != count:
             raise ValueError("%s: need a C-contiguous float64 array of %d elements" % (name, count))
         return out.ctypes.data, _lib.HOST
+
+    def _wait(self, t):
+        """what torch has queued on its current stream (the tensor's values,
+        readers of an output): the solver's stream does not wait for it"""
+        cuda = _torch().cuda
+        if not cuda.is_current_stream_capturing():
+            cuda.current_stream(t.device).synchronize()
 
     def _check_device(self, t, name):
         if t.device.index is not None and t.device.index != self.cfg.device:
