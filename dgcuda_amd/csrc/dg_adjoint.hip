@@ -581,8 +581,7 @@ __global__ __launch_bounds__((vjp_blk<PHYS, P, MODE>())) void k_vjp(const AdjArg
     for (int n = 0; n < N; n++)
 #pragma unroll
       for (int i = 0; i < NP; i++) gf[n * NP + i] = g[n][i];
-    if (a.gout) combine_store<N * NP>(a.gout, gf, a.scale, a.ot, a.oc, a.nout, K, e);
-    if (a.gout2) combine_store<N * NP>(a.gout2, gf, a.c2g, a.o2t, a.o2c, a.n2, K, e);
+    combine_store<N * NP>(a.gout, gf, a.scale, a.ot, a.oc, a.nout, K, e);
   }
   if constexpr (TE) {
     if (a.geps) {
@@ -605,7 +604,7 @@ __global__ __launch_bounds__((vjp_blk<PHYS, P, MODE>())) void k_vjp(const AdjArg
           const double wv = kPark ? s_w[n * NP + i][threadIdx.x] : sc[n] * lam_at(a, q, e);
           ew = fma(wv, gld(a.kst + q, e), ew);
         }
-      a.geps[e] += a.scale * (gz - ew * (Jme / a.dt));
+      a.geps[e] += gz - ew * (Jme / a.dt);
     }
   }
 }
@@ -730,6 +729,12 @@ __global__ __launch_bounds__(kQuadBlk, (P == 4 ? 2 : 1)) void k_vjp_q(const AdjA
   // there wait in its row, and the results come back through row side 0
   constexpr bool kLast = TC::NQ1 % 4 == 1;
   __shared__ double s_lo[kLast ? kQuadBlk : 1][3][4];
+  // the Runge-Kutta terms of the result, summed here at the start and added at
+  // the end (a thread's own column): in the epilogue they were a round trip
+  // per entry or, batched, spills (the kernel is at its register cap), and in
+  // a launch of their own (42 us beside this kernel's 161 on 131,072 elements
+  // at p = 4) two more passes over the result
+  __shared__ double s_rk[NP][kQuadBlk];
   for (int q = threadIdx.x; q < 3 * NP * NQ1; q += kQuadBlk) s_side[q] = TC::SIDE[q];
   __syncthreads();
   const int K = a.m.K;
@@ -739,6 +744,23 @@ __global__ __launch_bounds__(kQuadBlk, (P == 4 ? 2 : 1)) void k_vjp_q(const AdjA
   const bool act = e < K;
   const int ee = act ? e : K - 1;
 
+  {
+    double v[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++) v[i] = 0.;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      if (t < a.nout) {
+        const double *src = a.ot[t] + (size_t)(n * NP) * K;
+        const double x = a.oc[t];
+#pragma unroll
+        for (int i = 0; i < NP; i++) v[i] = fma(x, gld(src, ee + i * K), v[i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NP; i++) s_rk[i][threadIdx.x] = v[i];
+    asm volatile("" ::: "memory");
+  }
   double c[NP], w[NP], g[NP];
   const double sc = a.dt / gld(a.m.J, ee);
 #pragma unroll
@@ -1029,58 +1051,9 @@ __global__ __launch_bounds__(kQuadBlk, (P == 4 ? 2 : 1)) void k_vjp_q(const AdjA
   }
   __builtin_amdgcn_sched_barrier(0);
   if (!act) return;
-  // (the launcher passes no combination terms: k_combine adds them after,
-  // see launch_adjoint_rhs)
-  if (a.gout) {
 #pragma unroll
-    for (int i = 0; i < NP; i++) {
-      const size_t q = (size_t)(n * NP + i) * K;
-      double v = a.scale * g[i];
-#pragma unroll
-      for (int t = 0; t < 4; t++)
-        if (t < a.nout) v = fma(a.oc[t], gld(a.ot[t] + q, e), v);
-      gst_nt(a.gout + q, e, v);
-    }
-  }
-  if (a.gout2) {
-#pragma unroll
-    for (int i = 0; i < NP; i++) {
-      const size_t q = (size_t)(n * NP + i) * K;
-      double v = a.c2g * g[i];
-#pragma unroll
-      for (int t = 0; t < 4; t++)
-        if (t < a.n2) v = fma(a.o2c[t], gld(a.o2t[t] + q, e), v);
-      gst_nt(a.gout2 + q, e, v);
-    }
-  }
-}
-
-// The RK combination added to a stored c0 g: out = fma(oc[nt-1],
-// ot[nt-1], ... fma(oc[0], ot[0], out)), in the order the stage adjoint
-// kernels use, so the result is the same to the bit.  With `in` set the
-// start value is c0 * in (another output that holds g itself) instead of
-// out.  Block row y is coefficient row y (K entries), one thread per
-// element; an entry's loads are all requested before the first is used.
-struct CombArgs {
-  double *out;
-  const double *in;
-  double c0;
-  const double *ot[4];
-  double oc[4];
-  int nt, K;
-};
-__global__ __launch_bounds__(BLK) void k_combine(const CombArgs c) {
-  const int e = blockIdx.x * BLK + threadIdx.x;
-  if (e >= c.K) return;
-  const size_t q = (size_t)blockIdx.y * c.K;
-  double x[4];
-#pragma unroll
-  for (int t = 0; t < 4; t++) x[t] = t < c.nt ? gld(c.ot[t] + q, e) : 0.;
-  double v = c.in ? c.c0 * gld(c.in + q, e) : gld(c.out + q, e);
-#pragma unroll
-  for (int t = 0; t < 4; t++)
-    if (t < c.nt) v = fma(c.oc[t], x[t], v);
-  gst_nt(c.out + q, e, v);
+  for (int i = 0; i < NP; i++)
+    gst_nt(a.gout + (size_t)(n * NP + i) * K, e, fma(a.scale, g[i], s_rk[i][threadIdx.x]));
 }
 
 // The point-parallel VJP (dg_vjp_s.h) up to these many elements, by system
@@ -1124,37 +1097,8 @@ void launch_adjoint_rhs(int phys, int p, const AdjArgs &a, hipStream_t s) {
     // the linear systems take the transpose that does not read the state;
     // for the TE eps gradient the side terms go first (k_vjp sums them)
     if constexpr (stage_quad<ph, pp>()) {
-      // the four-lane kernel stores c0 g only and k_combine adds the RK
-      // terms: in its epilogue each term would be a round trip per entry
-      // (batching them there spills, the kernel being at its register cap)
-      // When both outputs are wanted and the first is g itself (scale 1, no
-      // terms), the second starts from c2g times the first: the kernel
-      // writes one array fewer.
-      const bool from_first = a.gout && a.gout2 && a.nout == 0 && a.scale == 1.0;
-      AdjArgs b = a;
-      b.nout = 0;
-      b.n2 = 0;
-      if (from_first) b.gout2 = nullptr;
       hipLaunchKernelGGL((k_vjp_q<ph, pp>), dim3(nblocks(a.m.K, kQuadBlk / 4)), dim3(kQuadBlk), 0,
-                         s, b);
-      auto comb = [&](double *out, const double *in, double c0, const double *const(&ot)[4],
-                      const double(&oc)[4], int nt) {
-        if (!out || (nt <= 0 && !in)) return;
-        CombArgs c;
-        c.out = out;
-        c.in = in;
-        c.c0 = c0;
-        for (int t = 0; t < 4; t++) {
-          c.ot[t] = ot[t];
-          c.oc[t] = oc[t];
-        }
-        c.nt = nt;
-        c.K = a.m.K;
-        hipLaunchKernelGGL(k_combine, dim3(nblocks(a.m.K, BLK), nvars_of(ph) * np_of(pp)),
-                           dim3(BLK), 0, s, c);
-      };
-      comb(a.gout, nullptr, 0., a.ot, a.oc, a.nout);
-      comb(a.gout2, from_first ? a.gout : nullptr, a.c2g, a.o2t, a.o2c, a.n2);
+                         s, a);
     } else if constexpr (ph == PH_TE) {
       if (a.geps)
         hipLaunchKernelGGL((k_eps_side<pp>), dim3(nblocks(a.m.S, BLK)), dim3(BLK), 0, s, a);

@@ -1696,19 +1696,22 @@ extern "C" int dg_adjoint_solve(dg_handle *h, int nsteps, double dt, int every, 
   const int nres = resident_segments(nsteps, every, nseg, sb, [&](int ns) {
     return ((size_t)ns * S + 1) * sb + (want_eps ? (size_t)ns * S * kst_b : 0);
   });
-  const int nrec = nseg - nres;  // segments 0 .. nrec - 1 are recomputed
   h->adj_resident = nres;
-  const size_t seg_stages = nrec > 0 ? (size_t)every * S : 0;
-  size_t need = adj_stride(sb) * (S + 3);
-  if (nrec > 0) need += adj_stride(sb) * (nrec + seg_stages + 1);
+  // Segments 0 .. nrec - 1 are recomputed.  The last one never is: the sweep
+  // starts there, so its forward pass leaves its stage data in the recompute's
+  // buffers (unless it is resident anyway).
+  const int nrec = nres ? nseg - nres : nseg - 1;
+  const size_t seg_stages = nres < nseg ? (size_t)every * S : 0;
+  size_t need = adj_stride(sb) * (S + 2 + nrec);
+  if (nres < nseg) need += adj_stride(sb) * (seg_stages + 1);
   if (want_eps)
     need += adj_stride(kst_b) * seg_stages + adj_stride(sizeof(double) * h->K) +
             adj_stride(2 * sizeof(double) * h->S);
   AdjWorkspace ws(h);
   if ((rc = ws.reserve(need)) != DG_OK) return rc;
-  ws.take(wk, S + 3, sb);
-  if (nrec > 0) {
-    ws.take(ck, nrec, sb);
+  ws.take(wk, S + 2, sb);
+  ws.take(ck, nrec, sb);
+  if (nres < nseg) {
     ws.take(store, seg_stages + 1, sb);
     if (want_eps) ws.take(kst, seg_stages, kst_b);
   }
@@ -1743,30 +1746,17 @@ extern "C" int dg_adjoint_solve(dg_handle *h, int nsteps, double dt, int every, 
   h->adj_fix_fired = 0;
 
   const bool tdep = bnd_time_dependent(h);
-  // ---- the launches of the reverse sweep (run after the forward pass
-  // below).  Per step, stage r (last to first) runs one VJP on
-  // the single array gk_r; the launch for stage r >= 1 also writes the next
-  // weight, gk_{r-1} = a_{r,r-1} l_r + b_{r-1} g + sum_{r' > r} a_{r',r-1} l_r'
-  // (own-element terms), and the launch for stage 0 writes the new g,
-  // g + sum_r l_r, into the other g buffer.  The last stage reads b_{S-1} g.
+  // ---- the launches of the reverse sweep (run after the forward pass below):
+  // per step, stage r (last to first) runs one VJP and writes one array, the
+  // weight that the next launch reads (L[r], own-element terms included); the
+  // launch for stage 0 writes the new g into the other g buffer.
   double *Gn = wk.bufs[S + 1];
-  double *GKb = L[0];  // gk_{r-1} (L[0] itself is never stored: stage 0 writes g)
-  double *GKa = wk.bufs[S + 2];
   // One segment's launches: re-run it from its first state (in stb[0]: the
   // checkpoint, or for a resident segment the forward pass's state) keeping
   // every stage input (record), then walk it backwards (walk).  Without
   // time-dependent boundary data the launches of a segment depend only on
   // its length and on which g buffer it starts from, so they are captured
   // once as a graph and replayed.
-  // a tableau with only the subdiagonal (RK4, midpoint RK2, SSP-RK2) lets
-  // the stage adjoints l_r be recovered from the weights w_{r-1} that are
-  // written anyway, so no l_r array is stored
-  bool subdiag = true;
-  for (int r = 1; r < S; r++) {
-    if (T.a[r][r - 1] == 0.) subdiag = false;
-    for (int c = 0; c + 1 < r; c++)
-      if (T.a[r][c] != 0.) subdiag = false;
-  }
   auto record = [&](int ns, AdjBuffers &stb, AdjBuffers &ksb) -> int {
     // positivity flags of the checkpoint; each step's last stage writes
     // those of the state it stores, as in the forward solve
@@ -1816,59 +1806,36 @@ extern "C" int dg_adjoint_solve(dg_handle *h, int nsteps, double dt, int every, 
           aa.kst = ksb.bufs[(size_t)s * S + r];
           aa.gzs = d_gzs;
         }
-        double *next = (r & 1) ? GKa : GKb;  // never the array this launch reads
-        if (subdiag) {
-          // w_{r-1} = b_{r-1} g + a_{r,r-1} l_r goes to L[r]; no l_r array
-          next = L[r];
-          aa.gout = r == 0 ? Gn : nullptr;
-          if (r >= 1) {
-            aa.gout2 = next;
-            aa.c2g = T.a[r][r - 1];
-            aa.n2 = 0;
-            if (T.b[r - 1] != 0.) {
-              aa.o2t[0] = G;
-              aa.o2c[0] = T.b[r - 1];
-              aa.n2 = 1;
-            }
-          } else {
-            // g <- g + sum_r l_r with l_{r+1} = (w_r - b_r g) / a_{r+1,r}
-            double cg = 1.;
-            for (int r2 = 0; r2 + 1 < S; r2++) cg -= T.b[r2] / T.a[r2 + 1][r2];
-            aa.ot[0] = G;
-            aa.oc[0] = cg;
-            for (int r2 = 0; r2 + 1 < S; r2++) {
-              aa.ot[r2 + 1] = L[r2 + 1];
-              aa.oc[r2 + 1] = 1. / T.a[r2 + 1][r2];
-            }
-            aa.nout = S;
+        auto term = [&](const double *x, double c) {
+          if (c == 0.) return;
+          aa.ot[aa.nout] = x;
+          aa.oc[aa.nout++] = c;
+        };
+        if (h->cfg.integrator == DG_SSPRK3) {
+          // the transpose of the stages as they run, u_r = A u_0 + B (u_{r-1}
+          // + k(u_{r-1})): lam is d/du_{r+1}, the output d/du_r
+          static const double A[3] = {0., 0.75, 1. / 3.}, B[3] = {1., 0.25, 2. / 3.};
+          aa.lc = B[r];
+          term(lam, B[r]);
+          if (r == 0) {
+            term(L[2], A[1]);
+            term(G, A[2]);
           }
         } else if (r >= 1) {
-          aa.gout2 = next;
-          aa.c2g = T.a[r][r - 1];
-          int n2 = 0;
-          if (T.b[r - 1] != 0.) {
-            aa.o2t[n2] = G;
-            aa.o2c[n2++] = T.b[r - 1];
-          }
-          for (int r2 = r + 1; r2 < S; r2++)
-            if (T.a[r2][r - 1] != 0.) {
-              aa.o2t[n2] = L[r2];
-              aa.o2c[n2++] = T.a[r2][r - 1];
-            }
-          aa.n2 = n2;
-        } else {  // g <- g + sum_r l_r
-          aa.ot[0] = G;
-          aa.oc[0] = 1.;
-          for (int r2 = 1; r2 < S; r2++) {
-            aa.ot[r2] = L[r2];
-            aa.oc[r2] = 1.;
-          }
-          aa.nout = S;
+          // tableaus with the subdiagonal only: w_{r-1} = b_{r-1} g + a_{r,r-1} l_r
+          aa.scale = T.a[r][r - 1];
+          term(G, T.b[r - 1]);
+        } else {
+          // g <- g + sum_r l_r with l_{r+1} = (w_r - b_r g) / a_{r+1,r}
+          double cg = 1.;
+          for (int r2 = 0; r2 + 1 < S; r2++) cg -= T.b[r2] / T.a[r2 + 1][r2];
+          term(G, cg);
+          for (int r2 = 0; r2 + 1 < S; r2++) term(L[r2 + 1], 1. / T.a[r2 + 1][r2]);
         }
         if (tdep)
           launch_bnd(phys, p, mesh_dev(h), h->ph, h->d_st, 0., 0, tn + dt + T.c[r] * dt, h->stream);
         launch_adjoint_rhs(phys, p, aa, h->stream);
-        lam = next;
+        lam = L[r];
         lcoef = 1.0;
       }
       std::swap(G, Gn);
@@ -1892,14 +1859,14 @@ extern "C" int dg_adjoint_solve(dg_handle *h, int nsteps, double dt, int every, 
       if (rc) return rc;
       continue;
     }
-    // a resident segment: the recompute's launches run here, from the
-    // current state, and their stage data stay for the sweep
+    // a segment that is not recomputed: the recompute's launches run here,
+    // from the current state, and their stage data stay for the sweep
     const double tseg = q * every * dt;
-    AdjBuffers &rs = rstore[q - nrec];
+    AdjBuffers &rs = nres ? rstore[q - nrec] : store;
     HIPCHK(h, hipMemcpyAsync(rs.bufs[0], h->d_c, sb, hipMemcpyDeviceToDevice, h->stream));
     if ((rc = write_state(h, tseg + dt, dt)) != DG_OK) return rc;
     refresh_bnd_fixed(h, tseg);
-    if ((rc = record(ns, rs, rkst[q - nrec])) != DG_OK) return rc;
+    if ((rc = record(ns, rs, nres ? rkst[q - nrec] : kst)) != DG_OK) return rc;
     HIPCHK(h, hipMemcpyAsync(h->d_c, rs.bufs[(size_t)ns * S], sb, hipMemcpyDeviceToDevice,
                              h->stream));
   }
@@ -1920,16 +1887,19 @@ extern "C" int dg_adjoint_solve(dg_handle *h, int nsteps, double dt, int every, 
   for (int q = nseg - 1; q >= 0; q--) {
     const int ns = std::min(every, nsteps - q * every);
     const double tseg = q * every * dt;
-    if (q >= nrec) {  // resident: the stage data are there; walk it (not captured)
-      if ((rc = walk(ns, tseg, rstore[q - nrec], rkst[q - nrec])) != DG_OK) return rc;
+    if (q >= nrec) {  // the stage data are there; walk it (not captured)
+      rc = nres ? walk(ns, tseg, rstore[q - nrec], rkst[q - nrec]) : walk(ns, tseg, store, kst);
+      if (rc != DG_OK) return rc;
       HIPCHK(h, hipGetLastError());
       continue;
     }
     HIPCHK(h, hipMemcpyAsync(store.bufs[0], ck.bufs[q], sb, hipMemcpyDeviceToDevice, h->stream));
     rc = write_state(h, tseg + dt, dt);
     if (rc) return rc;
-    if (tdep) {
-      refresh_bnd_fixed(h, tseg);
+    // (two segments at most replay nothing: an odd one starts the next from
+    // the other g buffer)
+    if (tdep || nrec <= 2) {
+      if (tdep) refresh_bnd_fixed(h, tseg);
       if ((rc = segment(ns, tseg))) return rc;
       HIPCHK(h, hipGetLastError());
       continue;

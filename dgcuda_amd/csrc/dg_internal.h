@@ -235,17 +235,9 @@ struct AdjArgs {
   const double *lam;  // adjoint of k is lc * lam, [N][NP][K]
   double lc;
   double *gout;       // output [N][NP][K]: scale * (dk/du)^T lam + sum_t oc[t] ot[t], t < nout
-                      // (nullptr: not written)
   const double *ot[4];
   double oc[4];
   int nout;
-  // optional second output (own-element terms only):
-  // gout2 = c2g * (dk/du)^T lam + sum_t o2c[t] o2t[t], t < n2
-  double *gout2;
-  double c2g;
-  const double *o2t[4];
-  double o2c[4];
-  int n2;
   // Maxwell TE eps gradient: geps [K] accumulates it (nullptr: not formed),
   // from the forward stage's k = dt L(us) (kst) and the per-side impedance
   // terms gzs [2][S] (left, right element) that k_eps_side writes

@@ -1,9 +1,8 @@
 // dg_vjp_s.h -- the right-hand side's vector-Jacobian product on small
 // meshes: a thread per point, then a thread per coefficient, as the small
 // mesh stage (dg_stage_s.h).  One launch does what the wide path does in up
-// to three: for Maxwell TE's permittivity gradient the side points also form
-// the impedance terms (k_eps_side), and for Euler p >= 4 the epilogue adds
-// the Runge-Kutta terms itself (k_combine), the registers being free here.
+// two: for Maxwell TE's permittivity gradient the side points also form the
+// impedance terms (k_eps_side).
 // Included by dg_adjoint.hip (the flux VJPs it uses are defined there).
 #pragma once
 
@@ -214,12 +213,9 @@ __global__ __launch_bounds__(kSmallT) void k_vjp_s(const AdjArgs a) {
       const int n = r / NP, i = r % NP;
       const size_t o = (size_t)r * K;
       // the combination arrays first: they are in flight during the sums
-      double x[4], y[4];
+      double x[4];
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        x[u] = a.gout && u < a.nout ? gld(a.ot[u] + o, ee) : 0.;
-        y[u] = a.gout2 && u < a.n2 ? gld(a.o2t[u] + o, ee) : 0.;
-      }
+      for (int u = 0; u < 4; u++) x[u] = u < a.nout ? gld(a.ot[u] + o, ee) : 0.;
       double g = 0.;
 #pragma unroll
       for (int j = 0; j < NQ; j++) g = fma(s_g[j][n][el], s_B[i * NQ + j], g);
@@ -228,14 +224,11 @@ __global__ __launch_bounds__(kSmallT) void k_vjp_s(const AdjArgs a) {
 #pragma unroll
         for (int j = 0; j < NQ1; j++)
           g = fma(s_f[k * NQ1 + j][n][el], s_side[(k * NP + i) * NQ1 + j], g);
-      double v = a.scale * g, v2 = a.c2g * g;
+      double v = a.scale * g;
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
+      for (int u = 0; u < 4; u++)
         if (u < a.nout) v = fma(a.oc[u], x[u], v);
-        if (u < a.n2) v2 = fma(a.o2c[u], y[u], v2);
-      }
-      if (act && a.gout) gst(a.gout + o, e, v);
-      if (act && a.gout2) gst(a.gout2 + o, e, v2);
+      if (act) gst(a.gout + o, e, v);
       if constexpr (EPS) {
         if (n < 2) s_k[r][el] = ow[q] * gld(a.kst + o, ee);
       }
@@ -250,7 +243,7 @@ __global__ __launch_bounds__(kSmallT) void k_vjp_s(const AdjArgs a) {
       for (int s = 0; s < NS; s++) gz += s_z[s][el];
       for (int r = 0; r < 2 * NP; r++) ew += s_k[r][el];
       const double z = sqrt(a.ph.mu / eps_me);
-      a.geps[e] += a.scale * (gz * (-z / (2. * eps_me)) - a.lc * ew / eps_me);
+      a.geps[e] += gz * (-z / (2. * eps_me)) - a.lc * ew / eps_me;
     }
   }
 }
