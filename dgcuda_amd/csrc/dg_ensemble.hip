@@ -219,6 +219,18 @@ void launch_finish_ens(DevState *st, const EnsInst *inst, int ninst, const EnsPa
   hipLaunchKernelGGL(k_finish_ens, dim3(ninst), dim3(BLK), 0, s, st, inst, parts, f);
 }
 
+__global__ __launch_bounds__(BLK) void k_rows(int n, double *dst, int dstride, const double *src,
+                                              int sstride) {
+  const int e = blockIdx.x * BLK + threadIdx.x;
+  if (e < n) dst[(size_t)blockIdx.y * dstride + e] = src[(size_t)blockIdx.y * sstride + e];
+}
+
+void launch_rows(int rows, int n, double *dst, int dstride, const double *src, int sstride,
+                 hipStream_t s) {
+  hipLaunchKernelGGL(k_rows, dim3(nblocks(n, BLK), rows), dim3(BLK), 0, s, n, dst, dstride, src,
+                     sstride);
+}
+
 int ens_vgprs(int phys, int B) {
   int v = -1;
   auto get = [&](const void *fn) {

@@ -187,6 +187,9 @@ void launch_bnd_ens(int phys, int p, const MeshDev &m, const PhysParams *ph, con
 void launch_finish_ens(DevState *st, const EnsInst *inst, int ninst, const EnsParts &parts,
                        const FinishArgs &f, hipStream_t s);
 int ens_vgprs(int phys, int B);
+// dst[r][0 .. n) = src[r][0 .. n) for rows of other strides
+void launch_rows(int rows, int n, double *dst, int dstride, const double *src, int sstride,
+                 hipStream_t s);
 
 // fixed scratch of dg_eval_rhs_noalloc (dg_kernels.hip): the DevState at
 // byte 0, the positivity flags ([K] ints, K <= kScratchMaxK) at byte 256

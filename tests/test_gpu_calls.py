@@ -98,3 +98,30 @@ def test_adjoint_solves_of_other_lengths_on_one_handle():
         s.set_objective(L.OBJ_PATCH_SQ, (0.1, 0.9, 0.1, 0.9, 2))
         assert np.isfinite(s.adjoint_solve(3, 1e-3)[1]).all()
         s.close()
+
+
+def test_ensemble_coefficients_on_the_device():
+    """an instance's rows go to and from a device array in one launch (sizes
+    around the 256-thread blocks and an odd 8-byte offset), as through the host"""
+    import torch
+    from dgcuda_amd.ensemble import Ensemble
+    E = Ensemble(physics=L.SWE, flux=L.FLUX_ROE, g=9.81, integrator=L.SSPRK3,
+                 problem=L.PROB_SWE_BUMP)
+    for n, p in ((4, 1), (11, 3), (12, 0), (16, 2)):
+        E.add(M.structured(n, periodic=False, jitter=0.2, seed=n), p,
+              (1.0, 0.1, 0.5, 0.5, 0.1, 1.0))
+    E.build()
+    before = [E.coeffs(i) for i in range(4)]
+    for i in range(4):
+        x = np.random.default_rng(i).standard_normal(before[i].shape)
+        d = torch.zeros(2 * x.size + 1, dtype=torch.float64, device="cuda")
+        d[1:x.size + 1] = torch.from_numpy(x).reshape(-1).cuda()
+        torch.cuda.synchronize()
+        a = d.data_ptr() + 8
+        assert E.lib.dg_ens_set_coeffs(E.e, i, ctypes.c_void_p(a), L.DEVICE) == 0
+        assert np.array_equal(E.coeffs(i), x)
+        a += 8 * x.size
+        assert E.lib.dg_ens_get_coeffs(E.e, i, ctypes.c_void_p(a), L.DEVICE) == 0
+        assert np.array_equal(d[1 + x.size:].cpu().numpy(), x.reshape(-1)) and d[0].item() == 0.0
+        for j in range(i + 1, 4):
+            assert np.array_equal(E.coeffs(j), before[j])
