@@ -1059,14 +1059,13 @@ __global__ __launch_bounds__(kQuadBlk, (P == 4 ? 2 : 1)) void k_vjp_q(const AdjA
 // The point-parallel VJP (dg_vjp_s.h) up to these many elements, by system
 // (the last row: TE with the permittivity gradient) and order.  As for the
 // stage, the wide kernels cost one wave's code below, and LDS reads bound the
-// point-parallel one above: us per stage of a reverse sweep (recompute
-// included), point-parallel against wide, on 968 / 8,192 / 32,768 elements:
-//   Euler p = 3    20 / 92    48 / 93    168 / 143
-//   Euler p = 4    25 / 41    65 / 60    226 / 133
-//   SWE Roe p = 3  17 / 79    31 / 79     90 / 105
-//   TM p = 5       18 / 133   53 / 151   172 / 257
-//   TE eps p = 3   16 / 35    30 / 42     89 / 61
-//   adv p = 1      12 / 13    12 / 13     17 / 15
+// point-parallel one above: us per stage of a reverse sweep (32 steps every 4,
+// recompute included), point-parallel / wide, at 968 elements and below the line:
+//   Euler p = 3    16 / 118    20,000:  70 / 105
+//   Euler p = 4    21 / 67      5,832:  38 / 50
+//   SWE Roe p = 3  14 / 90     40,328:  88 / 103
+//   TE p = 5       15 / 156    64,800: 198 / 226
+//   adv p = 1      9 / 13      12,168:  10 / 13
 static int small_max_vjp(int phys, int p, bool eps) {
   static constexpr int k[5][PMAX + 1] = {{32768, 12288, 16384, 16384, 16384, 10240},
                                          {32768, 24576, 20480, 20480, 6144, 4096},
@@ -1080,14 +1079,25 @@ void launch_adjoint_rhs(int phys, int p, const AdjArgs &a, hipStream_t s) {
   dispatch(phys, p, [&](auto PH, auto PP) {
     constexpr int ph = decltype(PH)::value, pp = decltype(PP)::value;
     if (a.m.K <= small_max_vjp(ph, pp, a.geps != nullptr)) {
-      const dim3 g(nblocks(a.m.K, small_eb(pp))), b(kSmallT);
-      if constexpr (ph == PH_TE) {
-        if (a.geps) {
-          hipLaunchKernelGGL((k_vjp_s<ph, pp, true>), g, b, 0, s, a);
+      const int nblk = nblocks(a.m.K, small_eb(pp));
+      auto small = [&](auto FULL) {
+        constexpr bool full = decltype(FULL)::value;
+        const dim3 g(nblk), b(small_t<ph, pp, full, true>());
+        if constexpr (ph == PH_TE) {
+          if (a.geps) {
+            hipLaunchKernelGGL((k_vjp_s<ph, pp, true, full>), g, b, 0, s, a);
+            return;
+          }
+        }
+        hipLaunchKernelGGL((k_vjp_s<ph, pp, false, full>), g, b, 0, s, a);
+      };
+      if constexpr (!small_full(pp, 1 << 30)) {
+        if (!small_full(pp, nblk)) {
+          small(std::false_type{});
           return;
         }
       }
-      hipLaunchKernelGGL((k_vjp_s<ph, pp, false>), g, b, 0, s, a);
+      small(std::true_type{});
       return;
     }
     auto go = [&](auto M) {

@@ -111,17 +111,18 @@ int small_blocks(int p, int K) { return nblocks(K, small_eb(p)); }
 // the one-thread (or four-lane) stage costs the instruction stream of a
 // single wave whatever the mesh: us per SSP-RK3 stage, the step's close
 // included, periodic meshes, point-parallel against the wide kernel:
-//   Euler p = 3    968: 8.1 / 32    8,192: 13.1 / 20.6   16,200: 22.2 / 20.9
-//   Euler p = 4    968: 10 / 33     4,050: 13 / 32        8,192: 18.2 / 17.5
-//   SWE Roe p = 3  968: 6.2 / 17   16,200: 16.9 / 17.8   32,768: 27.9 / 18.8
-//   TE p = 5       968: 7.4 / 76   16,200: 41 / 69       32,768: 77 / 71
-//   adv p = 1      968: 4.0 / 5.0   8,192: 4.5 / 5.0     16,200: 5.4 / 5.1
+//   Euler p = 3    968: 7.3 / 32   14,112: 20.4 / 21.2
+//   Euler p = 4    968: 9.8 / 33    6,050: 14.7 / 16.7
+//   SWE Roe p = 3  968: 6.5 / 18   16,200: 17.2 / 18.2
+//   TE p = 2       968: 5.8 / 11   16,200: 11.6 / 11.2
+//   TE p = 5       968: 7.1 / 77   28,322: 56 / 72
+//   adv p = 1      968: 4.2 / 5.3  12,168: 5.1 / 5.4
 // Above, the LDS table reads per multiply-add set its time (1.25 per
 // multiply-add with four variables, more with fewer), which the wide kernels
 // do not have.
 int small_max_k(int phys, int p) {
   static constexpr int k[3][PMAX + 1] = {{32768, 12288, 16384, 12288, 12288, 8192},
-                                         {32768, 16384, 16384, 16384, 20480, 28672},
+                                         {32768, 16384, 12288, 16384, 20480, 28672},
                                          {16384, 12288, 16384, 14336, 6144, 6144}};
   const int n = nvars_of(phys);
   return k[n == 1 ? 0 : n - 2][p];
@@ -133,14 +134,24 @@ void launch_stage(int phys, int p, const StageArgs &a0, hipStream_t s) {
     constexpr int ph = decltype(PH)::value, pp = decltype(PP)::value;
     if (a.small) {
       a.nblk = small_blocks(pp, a.m.K);
-      const dim3 g(a.nblk), b(kSmallT);
-      if constexpr (small_tdb<ph>()) {
-        if (a.tdb) {
-          hipLaunchKernelGGL((k_stage_s<ph, pp, true>), g, b, 0, s, a);
+      auto go = [&](auto FULL) {
+        constexpr bool full = decltype(FULL)::value;
+        const dim3 g(a.nblk), b(small_t<ph, pp, full>());
+        if constexpr (small_tdb<ph>()) {
+          if (a.tdb) {
+            hipLaunchKernelGGL((k_stage_s<ph, pp, true, full>), g, b, 0, s, a);
+            return;
+          }
+        }
+        hipLaunchKernelGGL((k_stage_s<ph, pp, false, full>), g, b, 0, s, a);
+      };
+      if constexpr (!small_full(pp, 1 << 30)) {
+        if (!small_full(pp, a.nblk)) {
+          go(std::false_type{});
           return;
         }
       }
-      hipLaunchKernelGGL((k_stage_s<ph, pp, false>), g, b, 0, s, a);
+      go(std::true_type{});
       return;
     }
     if constexpr (stage_quad<ph, pp>()) {

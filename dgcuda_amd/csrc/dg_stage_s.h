@@ -4,7 +4,7 @@
 // On a mesh of a few thousand elements the one-thread-per-element stage is a
 // single wave on a few CUs that walks tens of kilobytes of straight-line code
 // (every table entry an immediate), so its time is the instruction stream of
-// one wave and the chip idles.  Here a block of 256 threads takes EB elements:
+// one wave and the chip idles.  Here a block takes EB elements:
 //   load     the elements' own and their neighbours' coefficients into LDS,
 //            with every other operand (tables, metric, step base) in flight
 //   points   a thread per side or volume point: the states there, the
@@ -17,30 +17,82 @@
 // first stage of a step closes the step before it (every block reduces the
 // partials, block 0 stores the new step state), and time-dependent boundary
 // data are evaluated by the side points that use them.
-// Bound by latency (launch, two dependent memory round trips, LDS): rotating
-// hill p = 4 on 1,080 triangles 26.4 us per RK4 stage with its boundary and
-// close before, 6.6 us now; supersonic vortex p = 3 on 2,880 triangles 22.9 ->
-// 10.0 us (fewer elements per block fill more CUs, but below the widths here
-// the loads fall under 32 B per row).
+// Bound by latency: of 8.4 us per stage (supersonic vortex p = 3 on 2,880
+// triangles; 22.9 on the one-thread kernel with its boundary and close) 2.4 are
+// the launch, 2.6 the two dependent memory round trips and the store, the rest
+// the points, the modes and the positivity check.  Rotating hill p = 4 on 1,080
+// triangles: 26.4 -> 6.2 us.  (Fewer elements per block fill more CUs, but
+// below the widths here the loads fall under 32 B per row.)
 #pragma once
 
 #include "dg_stage.h"
 
 namespace dgk {
 
-// elements per block: the points (3 (p+1) side and n_q volume points each)
-// of EB elements fit the block's 256 threads
+// elements per block, and its threads: a thread per point, the side points in
+// whole waves of their own (a wave with both would run one's code after the
+// other's), and a thread per coefficient (a second pass over them for the last
+// few doubles the modes' latency).  us per SSP-RK3 stage, Euler: p = 3 with 320
+// threads for its 320 coefficients 8.8 on 2,888 triangles, with 256 9.6.  At
+// p = 4 the second pass is nearly full and 256 threads are better than 512
+// (6,050 triangles 14.6 / 17.2).  At p = 2 the separate waves and the single
+// pass (384 threads, FULL) are better while the chip has room for them (2,888:
+// 7.2, with 256 7.9) and worse once it is full (16,200: 15.4 / 13.5): FULL is
+// for up to two blocks per CU.  The VJP at Euler p = 5 keeps the second pass
+// too: its flux adjoint spills in the registers that 384 threads leave (3,872:
+// 104.9 us a reverse stage; 66.9).
 __host__ __device__ constexpr int small_eb(int p) {
   return p == 0 ? 64 : p <= 2 ? 16 : p <= 4 ? 8 : 4;
 }
-constexpr int kSmallT = 256;
+template <int P, bool FULL>
+__host__ __device__ constexpr int small_side_t() {  // threads before the volume points
+  constexpr int n = small_eb(P) * 3 * (P + 1);
+  return FULL ? (n + 63) / 64 * 64 : n;
+}
+template <int PHYS, int P, bool FULL, bool VJP = false>
+__host__ __device__ constexpr int small_t() {
+  constexpr int eb = small_eb(P), pts = small_side_t<P, FULL>() + eb * nq_of(P);
+  constexpr int rows = FULL && P != 4 && !(VJP && P == 5) ? eb * nvars_of(PHYS) * np_of(P) : 0;
+  return ((pts > rows ? pts : rows) + 63) / 64 * 64;
+}
+__host__ __device__ constexpr bool small_full(int p, int nblk) { return p != 2 || nblk <= 512; }
+
+// An element's variables lie together in LDS, in pairs that one 16-byte access
+// moves (three variables are padded to four): b64 accesses were most of the
+// points' time.
+template <int PHYS>
+__host__ __device__ constexpr int small_nv() {
+  return nvars_of(PHYS) == 1 ? 1 : 4;
+}
+template <int N, int NV>
+__device__ __forceinline__ void lds_get(const double (&s)[NV], double *v) {
+  if constexpr (NV == 1) {
+    v[0] = s[0];
+  } else {
+    const dbl2 a = *(const dbl2 *)&s[0], b = *(const dbl2 *)&s[2];
+    v[0] = a.x;
+    v[1] = a.y;
+    v[2] = b.x;
+    if constexpr (N == 4) v[3] = b.y;
+  }
+}
+template <int N, int NV>
+__device__ __forceinline__ void lds_put(double (&s)[NV], const double *v) {
+  if constexpr (NV == 1) {
+    s[0] = v[0];
+  } else {
+    *(dbl2 *)&s[0] = dbl2{v[0], v[1]};
+    *(dbl2 *)&s[2] = dbl2{v[2], N == 4 ? v[3] : 0.};
+  }
+}
 
 // needs_fix of the block's elements' new coefficients s_c (element-local
 // positivity): rows 0 .. N-1 bound one variable each and every thread of an
 // element takes the same decision from the bounds; where they do not settle
 // it (rare), each thread checks one of its element's points
 template <int PHYS, int P, int EB>
-__device__ __forceinline__ bool small_needs_fix(const PhysParams &ph, const double (*s_c)[EB],
+__device__ __forceinline__ bool small_needs_fix(const PhysParams &ph,
+                                                const double (*s_c)[EB][small_nv<PHYS>()],
                                                 const double *s_B, const double *s_side,
                                                 double (*s_md)[nvars_of(PHYS)][EB], int *s_bad,
                                                 int el, int row) {
@@ -50,8 +102,8 @@ __device__ __forceinline__ bool small_needs_fix(const PhysParams &ph, const doub
   if (row < N) {
     double d = 0.;
 #pragma unroll
-    for (int i = 1; i < NP; i++) d = fma(fabs(s_c[row * NP + i][el]), phi_bound<P>(i), d);
-    s_md[0][row][el] = s_c[row * NP][el] * TC::B[0];
+    for (int i = 1; i < NP; i++) d = fma(fabs(s_c[i][el][row]), phi_bound<P>(i), d);
+    s_md[0][row][el] = s_c[0][el][row] * TC::B[0];
     s_md[1][row][el] = d * (1. + margin);
   }
   if (row == 0) s_bad[el] = 0;
@@ -74,7 +126,7 @@ __device__ __forceinline__ bool small_needs_fix(const PhysParams &ph, const doub
 #pragma unroll 1
     for (int i = 0; i < NP; i++)
 #pragma unroll
-      for (int n = 0; n < N; n++) U[n] = fma(s_c[n * NP + i][el], t[i * st], U[n]);
+      for (int n = 0; n < N; n++) U[n] = fma(s_c[i][el][n], t[i * st], U[n]);
     if (!is_physical<PHYS>(ph, U)) s_bad[el] = 1;  // (every writer stores the same value)
   }
   __syncthreads();
@@ -94,18 +146,20 @@ __host__ __device__ constexpr bool small_tdb() {
 // closes the pending step and stores slot 1; the later stages read slot 1;
 // the last one stores it back to slot 0 as pending.  No launch reads a slot
 // that it writes.
-template <int PHYS, int P, bool TDB>
-__global__ __launch_bounds__(kSmallT) void k_stage_s(const StageArgs a) {
+template <int PHYS, int P, bool TDB, bool FULL>
+__global__ __launch_bounds__((small_t<PHYS, P, FULL>())) void k_stage_s(const StageArgs a) {
   using TC = TabC<P>;
   constexpr int NP = TC::NP, NQ = TC::NQ, NQ1 = TC::NQ1, N = nvars_of(PHYS);
-  constexpr int EB = small_eb(P), NR = N * NP, NS = 3 * NQ1, T = kSmallT;
+  constexpr int EB = small_eb(P), NR = N * NP, NS = 3 * NQ1, T = small_t<PHYS, P, FULL>();
   constexpr int RW = T / EB;                 // rows of one pass over the elements
   constexpr int R = (NR + RW - 1) / RW;      // passes over the own rows
   constexpr int RN = (3 * NR + RW - 1) / RW;  // and over the neighbours'
-  static_assert(EB * (NS + NQ) <= T, "a thread per point");
-  __shared__ double s_B[NP * NQ], s_GX[NP * NQ], s_GY[NP * NQ], s_side[3 * NP * NQ1];
-  __shared__ double s_c[NR][EB], s_n[3 * NR][EB];
-  __shared__ double s_f[NS][N][EB], s_g[NQ][2][N][EB];
+  constexpr int SV = small_side_t<P, FULL>();  // the first volume point's thread
+  static_assert(SV + EB * NQ <= T && SV % EB == 0 && NQ + NS <= RW, "a thread per point");
+  constexpr int NV = small_nv<PHYS>();
+  __shared__ double s_B[NP * NQ], s_side[3 * NP * NQ1];
+  __shared__ dbl2 s_G[NP * NQ], s_g[NQ][N][EB];  // (r, s) components
+  __shared__ __align__(16) double s_c[NP][EB][NV], s_n[3][NP][EB][NV], s_f[NS][EB][NV];
   __shared__ double s_md[2][N][EB];
   __shared__ int s_bad[EB];
   __shared__ unsigned long long s_l[T / 64], s_k[T / 64];
@@ -130,9 +184,9 @@ __global__ __launch_bounds__(kSmallT) void k_stage_s(const StageArgs a) {
     const int r = row + q * RW, rr = r < 3 * NR ? r : 0;
     nbq[q] = a.m.slot[(size_t)(rr / NR) * K + ee].x;
   }
-  const bool is_side = t < EB * NS, is_vol = !is_side && t < EB * (NS + NQ);
+  const bool is_side = t < EB * NS, is_vol = t >= SV && t < SV + EB * NQ;
   const int sp = is_side ? row : 0, sk = sp / NQ1, jj = sp - sk * NQ1;
-  const int vj = is_vol ? row - NS : 0;
+  const int vj = is_vol ? row - SV / EB : 0;
   int2 sl = a.m.slot[(size_t)sk * K + ee];
   const double xr = gld(a.m.xr, ee), yr = gld(a.m.yr, ee);
   const double xs = gld(a.m.xs, ee), ys = gld(a.m.ys, ee);
@@ -156,7 +210,7 @@ __global__ __launch_bounds__(kSmallT) void k_stage_s(const StageArgs a) {
   }
   // the step state; the first stage of a step closes the step before it
   DevState S = a.st[(a.step_pos == STEP_MID || a.step_pos == STEP_LAST) ? 1 : 0];
-  constexpr int kU = kSmallFold / T;
+  constexpr int kU = (kSmallFold + T - 1) / T;
   unsigned long long pl[kU], pc[kU];
 #pragma unroll
   for (int u = 0; u < kU; u++) {
@@ -169,40 +223,49 @@ __global__ __launch_bounds__(kSmallT) void k_stage_s(const StageArgs a) {
   }
   for (int q = t; q < NP * NQ; q += T) {
     s_B[q] = TC::B[q];
-    s_GX[q] = TC::GX[q];
-    s_GY[q] = TC::GY[q];
+    s_G[q] = dbl2{TC::GX[q], TC::GY[q]};
   }
   for (int q = t; q < 3 * NP * NQ1; q += T) s_side[q] = TC::SIDE[q];
 
-  // ---- the neighbours' coefficients and this point's side
+  // ---- the neighbours' coefficients and this point's side, requested
+  // together: no branch lies between the loads (a row past the last, a
+  // boundary's missing neighbour have stand-ins), as
+  // each would make its load a round trip of its own
+  const int sid = sl.y >> 3;
+  double nbv[RN];
+  int fl_nb[RN];
 #pragma unroll
   for (int q = 0; q < RN; q++) {
-    const int r = row + q * RW;
-    if (r < 3 * NR) {
-      const int nr = r % NR;
-      double v = 0.;
-      if (nbq[q] >= 0) {
-        v = gld(a.us + (size_t)nr * K, nbq[q]);
-        // a flagged neighbour contributes its means only
-        if constexpr (has_positivity<PHYS>()) {
-          if (a.fix_in && nr % NP != 0 && gld_int(a.bad, nbq[q])) v = 0.;
-        }
-      }
-      s_n[r][el] = v;
+    const int r = row + q * RW, nr = r < 3 * NR ? r % NR : 0;
+    const int nb = nbq[q] >= 0 ? nbq[q] : ee;
+    nbv[q] = gld(a.us + (size_t)nr * K, nb);
+    fl_nb[q] = 0;
+  }
+  if constexpr (has_positivity<PHYS>()) {
+    if (a.fix_in) {
+#pragma unroll
+      for (int q = 0; q < RN; q++) fl_nb[q] = gld_int(a.bad, nbq[q] >= 0 ? nbq[q] : ee);
     }
   }
   double nx = 0., ny = 0., len = 0., bv[NMAX] = {0., 0., 0., 0.};
   if (is_side) {
-    const int sid = sl.y >> 3;
     nx = gld(a.m.snx, sid);
     ny = gld(a.m.sny, sid);
     len = gld(a.m.slen, sid);
-    if constexpr (PHYS == PH_TE) eps_nb = sl.x >= 0 ? gld(a.m.eps, sl.x) : eps_me;
+    const int bslot = a.m.side[sid].w;
+    if constexpr (PHYS == PH_TE) eps_nb = gld(a.m.eps, sl.x >= 0 ? sl.x : ee);
     if (sl.x < 0 && !(TDB && sl.x != -1)) {
-      const double *b = a.m.bnd_val + ((size_t)a.m.side[sid].w * NQ1 + jj) * NMAX;
+      const double *b = a.m.bnd_val + ((size_t)bslot * NQ1 + jj) * NMAX;
 #pragma unroll
       for (int n = 0; n < N; n++) bv[n] = b[n];
     }
+  }
+#pragma unroll
+  for (int q = 0; q < RN; q++) {
+    const int r = row + q * RW, nr = r % NR;
+    // a flagged neighbour contributes its means only
+    const bool zero = nbq[q] < 0 || (fl_nb[q] && nr % NP != 0);
+    if (r < 3 * NR) s_n[r / NR][nr % NP][el][nr / NP] = zero ? 0. : nbv[q];
   }
 #pragma unroll
   for (int q = 0; q < R; q++) {
@@ -210,7 +273,7 @@ __global__ __launch_bounds__(kSmallT) void k_stage_s(const StageArgs a) {
     if constexpr (has_positivity<PHYS>()) {
       if (a.fix_in && fl_me && r % NP != 0) own[q] = 0.;
     }
-    if (r < NR) s_c[r][el] = own[q];
+    if (r < NR) s_c[r % NP][el][r / NP] = own[q];
   }
   if (a.step_pos == STEP_FIRST) {
     unsigned long long kl = pl[0], kc = pc[0];
@@ -265,17 +328,15 @@ __global__ __launch_bounds__(kSmallT) void k_stage_s(const StageArgs a) {
     const double *po = s_side + (size_t)(sk * NP) * NQ1 + jj;
     const double *pn = s_side + (size_t)(nbls * NP) * NQ1 + NQ1 - 1 - jj;
 #pragma unroll
-    for (int n = 0; n < N; n++) {
-      Um[n] = s_c[n * NP][el] * po[0];
-      Un[n] = s_n[sk * NR + n * NP][el] * pn[0];
-    }
-#pragma unroll
-    for (int i = 1; i < NP; i++) {
+    for (int i = 0; i < NP; i++) {
       const double x = po[i * NQ1], y = pn[i * NQ1];
+      double cm[N], cn[N];
+      lds_get<N>(s_c[i][el], cm);
+      lds_get<N>(s_n[sk][i][el], cn);
 #pragma unroll
       for (int n = 0; n < N; n++) {
-        Um[n] = fma(s_c[n * NP + i][el], x, Um[n]);
-        Un[n] = fma(s_n[sk * NR + n * NP + i][el], y, Un[n]);
+        Um[n] = i ? fma(cm[n], x, Um[n]) : cm[n] * x;
+        Un[n] = i ? fma(cn[n], y, Un[n]) : cn[n] * y;
       }
     }
     if (nb < 0) {
@@ -315,17 +376,18 @@ __global__ __launch_bounds__(kSmallT) void k_stage_s(const StageArgs a) {
       f = (role ? 0.5 : -0.5) * len * w1;
     }
 #pragma unroll
-    for (int n = 0; n < N; n++) s_f[sp][n][el] = F[n] * f;
+    for (int n = 0; n < N; n++) F[n] *= f;
+    lds_put<N>(s_f[sp][el], F);
   } else if (is_vol) {
     // eval_volume conserv_kernels.cu:1042-1081 at point vj
     double U[NMAX], ga[NMAX], gb[NMAX];
 #pragma unroll
-    for (int n = 0; n < N; n++) U[n] = s_c[n * NP][el] * s_B[vj];
-#pragma unroll
-    for (int i = 1; i < NP; i++) {
+    for (int i = 0; i < NP; i++) {
       const double x = s_B[i * NQ + vj];
+      double cm[N];
+      lds_get<N>(s_c[i][el], cm);
 #pragma unroll
-      for (int n = 0; n < N; n++) U[n] = fma(s_c[n * NP + i][el], x, U[n]);
+      for (int n = 0; n < N; n++) U[n] = i ? fma(cm[n], x, U[n]) : cm[n] * x;
     }
     PhysParams pv = a.ph;
     if constexpr (PHYS == PH_ADV) {
@@ -337,10 +399,7 @@ __global__ __launch_bounds__(kSmallT) void k_stage_s(const StageArgs a) {
     }
     flux_contra<PHYS>(pv, U, xr, yr, xs, ys, ga, gb);
 #pragma unroll
-    for (int n = 0; n < N; n++) {
-      s_g[vj][0][n][el] = ga[n];
-      s_g[vj][1][n][el] = gb[n];
-    }
+    for (int n = 0; n < N; n++) s_g[vj][n][el] = dbl2{ga[n], gb[n]};
   }
   __syncthreads();
 
@@ -355,10 +414,12 @@ __global__ __launch_bounds__(kSmallT) void k_stage_s(const StageArgs a) {
     for (int k = 0; k < 3; k++)
 #pragma unroll
       for (int j = 0; j < NQ1; j++)
-        acc = fma(s_f[k * NQ1 + j][n][el], s_side[(k * NP + i) * NQ1 + j], acc);
+        acc = fma(s_f[k * NQ1 + j][el][n], s_side[(k * NP + i) * NQ1 + j], acc);
 #pragma unroll
-    for (int j = 0; j < NQ; j++)
-      acc = fma(s_GX[i * NQ + j], s_g[j][0][n][el], fma(s_GY[i * NQ + j], s_g[j][1][n][el], acc));
+    for (int j = 0; j < NQ; j++) {
+      const dbl2 G = s_G[i * NQ + j], g = s_g[j][n][el];
+      acc = fma(G.x, g.x, fma(G.y, g.y, acc));
+    }
     double sc = sdt;
     if constexpr (PHYS == PH_TE) sc = sdt * (n < 2 ? 1. / eps_me : 1. / a.ph.mu);
     acc *= sc;
@@ -393,7 +454,7 @@ __global__ __launch_bounds__(kSmallT) void k_stage_s(const StageArgs a) {
 #pragma unroll
     for (int q = 0; q < R; q++) {
       const int r = row + q * RW;
-      if (r < NR) s_c[r][el] = o[q];  // (read last before the barrier above)
+      if (r < NR) s_c[r % NP][el][r / NP] = o[q];  // (read last before the barrier above)
     }
     __syncthreads();
   }
@@ -431,7 +492,7 @@ __global__ __launch_bounds__(kSmallT) void k_stage_s(const StageArgs a) {
     if (a.cfl_mode && act && row == 0) {
       double U[NMAX];
 #pragma unroll
-      for (int n = 0; n < N; n++) U[n] = s_c[n * NP][el] * TC::B[0];
+      for (int n = 0; n < N; n++) U[n] = s_c[0][el][n] * TC::B[0];
       PhysParams pv = a.ph;
       if constexpr (PHYS == PH_ADV) {
         if (vary) {

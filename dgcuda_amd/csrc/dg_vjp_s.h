@@ -10,18 +10,20 @@
 
 namespace dgk {
 
-template <int PHYS, int P, bool EPS>
-__global__ __launch_bounds__(kSmallT) void k_vjp_s(const AdjArgs a) {
+template <int PHYS, int P, bool EPS, bool FULL>
+__global__ __launch_bounds__((small_t<PHYS, P, FULL, true>())) void k_vjp_s(const AdjArgs a) {
   using TC = TabC<P>;
   constexpr int NP = TC::NP, NQ = TC::NQ, NQ1 = TC::NQ1, N = nvars_of(PHYS);
   constexpr bool TE = PHYS == PH_TE;
   constexpr bool kU = EPS || !linear_flux<PHYS>();  // the state is read
-  constexpr int EB = small_eb(P), NR = N * NP, NS = 3 * NQ1, T = kSmallT;
+  constexpr int EB = small_eb(P), NR = N * NP, NS = 3 * NQ1, T = small_t<PHYS, P, FULL, true>();
   constexpr int RW = T / EB, R = (NR + RW - 1) / RW, RN = (3 * NR + RW - 1) / RW;
-  constexpr int RU = kU ? NR : 1;
-  __shared__ double s_B[NP * NQ], s_GX[NP * NQ], s_GY[NP * NQ], s_side[3 * NP * NQ1];
-  __shared__ double s_w[NR][EB], s_nw[3 * NR][EB], s_u[RU][EB], s_nu[3 * RU][EB];
-  __shared__ double s_f[NS][N][EB], s_g[NQ][N][EB];
+  constexpr int NV = small_nv<PHYS>(), NPU = kU ? NP : 1;
+  __shared__ double s_B[NP * NQ], s_side[3 * NP * NQ1];
+  __shared__ dbl2 s_G[NP * NQ];
+  __shared__ __align__(16) double s_w[NP][EB][NV], s_nw[3][NP][EB][NV];
+  __shared__ __align__(16) double s_u[NPU][EB][NV], s_nu[3][NPU][EB][NV];
+  __shared__ __align__(16) double s_f[NS][EB][NV], s_g[NQ][EB][NV];
   __shared__ double s_z[EPS ? NS : 1][EB], s_k[EPS ? 2 * NP : 1][EB];
   const int t = threadIdx.x, el = t % EB, row = t / EB;
   const int K = a.m.K;
@@ -36,9 +38,10 @@ __global__ __launch_bounds__(kSmallT) void k_vjp_s(const AdjArgs a) {
     const int r = row + q * RW, rr = r < 3 * NR ? r : 0;
     nbq[q] = a.m.slot[(size_t)(rr / NR) * K + ee].x;
   }
-  const bool is_side = t < EB * NS, is_vol = !is_side && t < EB * (NS + NQ);
+  constexpr int SV = small_side_t<P, FULL>();  // the first volume point's thread
+  const bool is_side = t < EB * NS, is_vol = t >= SV && t < SV + EB * NQ;
   const int sp = is_side ? row : 0, sk = sp / NQ1, jj = sp - sk * NQ1;
-  const int vj = is_vol ? row - NS : 0;
+  const int vj = is_vol ? row - SV / EB : 0;
   const int2 sl = a.m.slot[(size_t)sk * K + ee];
   double ow[R], ou[R];
 #pragma unroll
@@ -61,44 +64,49 @@ __global__ __launch_bounds__(kSmallT) void k_vjp_s(const AdjArgs a) {
   }
   for (int q = t; q < NP * NQ; q += T) {
     s_B[q] = TC::B[q];
-    s_GX[q] = TC::GX[q];
-    s_GY[q] = TC::GY[q];
+    s_G[q] = dbl2{TC::GX[q], TC::GY[q]};
   }
   for (int q = t; q < 3 * NP * NQ1; q += T) s_side[q] = TC::SIDE[q];
+  // the neighbours and this point's side, no branch between the loads (as the
+  // stage's)
+  const int sid = sl.y >> 3;
+  double nw[RN], nu[RN];
 #pragma unroll
   for (int q = 0; q < RN; q++) {
-    const int r = row + q * RW;
-    if (r < 3 * NR) {
-      const bool has = nbq[q] >= 0;
-      const int nb = has ? nbq[q] : ee;
-      const double w = gld(a.lam + (size_t)(r % NR) * K, nb);
-      s_nw[r][el] = has ? w : 0.;
-      if constexpr (kU) {
-        const double u = gld(a.us + (size_t)(r % NR) * K, nb);
-        s_nu[r][el] = has ? u : 0.;
-      }
-    }
+    const int r = row + q * RW, nr = r < 3 * NR ? r % NR : 0, nb = nbq[q] >= 0 ? nbq[q] : ee;
+    nw[q] = gld(a.lam + (size_t)nr * K, nb);
+    nu[q] = 0.;
+    if constexpr (kU) nu[q] = gld(a.us + (size_t)nr * K, nb);
   }
   double nx = 0., ny = 0., len = 0., Jnb = 1., bv[NMAX] = {0., 0., 0., 0.};
   if (is_side) {
-    const int sid = sl.y >> 3;
     nx = gld(a.m.snx, sid);
     ny = gld(a.m.sny, sid);
     len = gld(a.m.slen, sid);
-    Jnb = gld(a.m.J, sl.x >= 0 ? sl.x : ee);
-    if constexpr (TE) eps_nb = sl.x >= 0 ? gld(a.m.eps, sl.x) : eps_me;
+    const int snb_e = sl.x >= 0 ? sl.x : ee, bslot = a.m.side[sid].w;
+    Jnb = gld(a.m.J, snb_e);
+    if constexpr (TE) eps_nb = gld(a.m.eps, snb_e);
     if (sl.x < 0) {
-      const double *b = a.m.bnd_val + ((size_t)a.m.side[sid].w * NQ1 + jj) * NMAX;
+      const double *b = a.m.bnd_val + ((size_t)bslot * NQ1 + jj) * NMAX;
 #pragma unroll
       for (int n = 0; n < NMAX; n++) bv[n] = b[n];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < RN; q++) {
+    const int r = row + q * RW, nr = r % NR;
+    const bool has = nbq[q] >= 0;
+    if (r < 3 * NR) {
+      s_nw[r / NR][nr % NP][el][nr / NP] = has ? nw[q] : 0.;
+      if constexpr (kU) s_nu[r / NR][nr % NP][el][nr / NP] = has ? nu[q] : 0.;
     }
   }
 #pragma unroll
   for (int q = 0; q < R; q++) {
     const int r = row + q * RW;
     if (r < NR) {
-      s_w[r][el] = ow[q];
-      if constexpr (kU) s_u[r][el] = ou[q];
+      s_w[r % NP][el][r / NP] = ow[q];
+      if constexpr (kU) s_u[r % NP][el][r / NP] = ou[q];
     }
   }
   // the weights' scale dt / J (TE also 1/eps, 1/mu per row), times lc
@@ -120,13 +128,20 @@ __global__ __launch_bounds__(kSmallT) void k_vjp_s(const AdjArgs a) {
 #pragma unroll
     for (int i = 0; i < NP; i++) {
       const double x = po[i * NQ1], y = pn[i * NQ1];
+      double wm[N], wn[N], um[N], un[N];
+      lds_get<N>(s_w[i][el], wm);
+      lds_get<N>(s_nw[sk][i][el], wn);
+      if constexpr (kU) {
+        lds_get<N>(s_u[i][el], um);
+        lds_get<N>(s_nu[sk][i][el], un);
+      }
 #pragma unroll
       for (int n = 0; n < N; n++) {
-        Wm[n] = fma(s_w[n * NP + i][el], x, Wm[n]);
-        Wn[n] = fma(s_nw[sk * NR + n * NP + i][el], y, Wn[n]);
+        Wm[n] = fma(wm[n], x, Wm[n]);
+        Wn[n] = fma(wn[n], y, Wn[n]);
         if constexpr (kU) {
-          Um[n] = fma(s_u[n * NP + i][el], x, Um[n]);
-          Un[n] = fma(s_nu[sk * NR + n * NP + i][el], y, Un[n]);
+          Um[n] = fma(um[n], x, Um[n]);
+          Un[n] = fma(un[n], y, Un[n]);
         }
       }
     }
@@ -165,8 +180,7 @@ __global__ __launch_bounds__(kSmallT) void k_vjp_s(const AdjArgs a) {
 #pragma unroll
     for (int n = 0; n < N; n++) gme[n] = role ? gR[n] : gL[n];
     if (nb == -1) wall_vjp<PHYS>(a.ph, bv[0], bv[1], bv[2], gR, gme);
-#pragma unroll
-    for (int n = 0; n < N; n++) s_f[sp][n][el] = gme[n];
+    lds_put<N>(s_f[sp][el], gme);
     // a boundary's ghost state carries the element's own impedance
     if constexpr (EPS) s_z[sp][el] = nb < 0 ? gzl + gzr : (role ? gzr : gzl);
   } else if (is_vol) {
@@ -176,12 +190,15 @@ __global__ __launch_bounds__(kSmallT) void k_vjp_s(const AdjArgs a) {
     for (int n = 0; n < N; n++) wa[n] = wb[n] = 0.;
 #pragma unroll
     for (int i = 0; i < NP; i++) {
-      const double gx = s_GX[i * NQ + vj], gy = s_GY[i * NQ + vj], ph = s_B[i * NQ + vj];
+      const dbl2 G = s_G[i * NQ + vj];
+      double wm[N], um[N];
+      lds_get<N>(s_w[i][el], wm);
+      if constexpr (kU) lds_get<N>(s_u[i][el], um);
 #pragma unroll
       for (int n = 0; n < N; n++) {
-        wa[n] = fma(s_w[n * NP + i][el], gx, wa[n]);
-        wb[n] = fma(s_w[n * NP + i][el], gy, wb[n]);
-        if constexpr (kU) U[n] = fma(s_u[n * NP + i][el], ph, U[n]);
+        wa[n] = fma(wm[n], G.x, wa[n]);
+        wb[n] = fma(wm[n], G.y, wb[n]);
+        if constexpr (kU) U[n] = fma(um[n], s_B[i * NQ + vj], U[n]);
       }
     }
 #pragma unroll
@@ -200,8 +217,7 @@ __global__ __launch_bounds__(kSmallT) void k_vjp_s(const AdjArgs a) {
     }
     fn_vjp<PHYS>(pv, U, 1.0, 0.0, gfx, gU);
     fn_vjp<PHYS>(pv, U, 0.0, 1.0, gfy, gU);
-#pragma unroll
-    for (int n = 0; n < N; n++) s_g[vj][n][el] = gU[n];
+    lds_put<N>(s_g[vj][el], gU);
   }
   __syncthreads();
 
@@ -218,12 +234,12 @@ __global__ __launch_bounds__(kSmallT) void k_vjp_s(const AdjArgs a) {
       for (int u = 0; u < 4; u++) x[u] = u < a.nout ? gld(a.ot[u] + o, ee) : 0.;
       double g = 0.;
 #pragma unroll
-      for (int j = 0; j < NQ; j++) g = fma(s_g[j][n][el], s_B[i * NQ + j], g);
+      for (int j = 0; j < NQ; j++) g = fma(s_g[j][el][n], s_B[i * NQ + j], g);
 #pragma unroll
       for (int k = 0; k < 3; k++)
 #pragma unroll
         for (int j = 0; j < NQ1; j++)
-          g = fma(s_f[k * NQ1 + j][n][el], s_side[(k * NP + i) * NQ1 + j], g);
+          g = fma(s_f[k * NQ1 + j][el][n], s_side[(k * NP + i) * NQ1 + j], g);
       double v = a.scale * g;
 #pragma unroll
       for (int u = 0; u < 4; u++)
