@@ -54,7 +54,9 @@ struct DevState {
 };
 
 enum StageMode { M_KONLY = 0, M_US_CK = 1, M_A_UN_B_US_CK = 2, M_UN_CK = 3 };
-enum AccMode { ACC_NONE = 0, ACC_SET6 = 1, ACC_ADD3 = 2, ACC_FINAL6 = 3 };
+// ACC_STAGES: RK4's last stage from the stage states themselves (no positivity
+// fix has touched them): u + ((u1 - u) + 2 (u2 - u) + (u3 - u)) / 3 + k4 / 6
+enum AccMode { ACC_NONE = 0, ACC_SET6 = 1, ACC_ADD3 = 2, ACC_FINAL6 = 3, ACC_STAGES = 4 };
 
 // where a small-mesh stage stands in its step (k_stage_s); STEP_NONE: the
 // step is closed by a launch of its own (or there is none)
@@ -87,6 +89,7 @@ struct StageArgs {
   const double *un;  // step base    [N][NP][K]
   double *out;       // stage output
   double *acc;       // RK4 running combination
+  const double *u1, *u2;  // ACC_STAGES: the inputs of the second and third stage
   DevState *st;
   PhysParams ph;
   int mode, accmode;

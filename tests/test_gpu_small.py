@@ -173,3 +173,24 @@ def test_limited_steps_either_side_of_the_size_rule(physics, integrator, K):
         assert rc == 0 and n == no and abs(t - to) <= 1e-13 * to and r < TOL
         assert "conv_tol" not in kw or abs(c - co) <= 1e-10 * abs(co)
     s.close()
+
+
+@pytest.mark.parametrize("physics,p,K", [
+    (L.MAXWELL_TE, 3, 578), (L.MAXWELL_TE, 3, 17298), (L.MAXWELL_TE, 4, 20808),
+    (L.MAXWELL_TM, 5, 29282), (L.MAXWELL_TM, 1, 16928), (L.ADVECTION, 0, 33282),
+    (L.ADVECTION, 2, 16928), (L.ADVECTION, 5, 8978)])
+def test_rk4_from_its_stage_states(physics, p, K):
+    """RK4 without a running combination (systems without a positivity fix),
+    on the point-parallel and the one-thread kernel, with the step-to-step
+    change that the last stage forms beside its store"""
+    s, o = _pair(physics, p, K, periodic=True, integrator=L.RK4, cfl=0.3)
+    print("rk4 physics", physics, "p", p, "K", s.K, flush=True)
+    t, dt = s.step(3)
+    rc, to, dto = o.run(3)
+    assert rc == 0 and abs(t - to) <= 1e-13 * to and rel_l2(s.coeffs(), o.coeffs()) < TOL
+    t, n, c = s.run(t=t, max_steps=3, conv_tol=0.0)
+    rc, to, no, co, _ = o.run_until(t0=to, max_steps=3, conv_tol=0.0)
+    r = rel_l2(s.coeffs(), o.coeffs())
+    print("  rel", r, "change", c, co)
+    assert rc == 0 and n == no and r < TOL and abs(c - co) <= 1e-10 * abs(co)
+    s.close()
