@@ -72,6 +72,7 @@ struct dg_handle {
   unsigned long long *d_part = nullptr;  // per-block maxima of the step reduction
   char *d_ws = nullptr;                  // dg_adjoint_solve's buffers, kept for the next call
   size_t ws_bytes = 0;
+  bool ws_busy = false;                  // a solve is using them
   double *d_red = nullptr;               // [kSumBlocks + 1] objective sum: partials, result
   double *d_gu = nullptr;                // dg_adjoint_rhs's output before its copy out
   int *d_bad = nullptr;                  // positivity flags of the stored state d_c
@@ -119,7 +120,7 @@ static int alloc(dg_handle *h, void **p, size_t bytes) {
     *p = nullptr;
   }
   hipError_t e = hipMalloc(p, bytes ? bytes : 8);
-  if (e != hipSuccess && h->d_ws && *p != h->d_ws) {  // the kept adjoint buffers go first
+  if (e != hipSuccess && h->d_ws && !h->ws_busy) {  // the kept adjoint buffers go first
     (void)hipGetLastError();
     (void)hipFree(h->d_ws);
     h->d_ws = nullptr;
@@ -1474,9 +1475,9 @@ Butcher butcher_of(int integ) {
 
 // Device buffers of the adjoint: a group's buffers lie at 256-byte-aligned
 // offsets, each 8 KiB past a 256-byte multiple of the one before.  With the
-// 8 KiB pad the config-5 sweep ran 1.8 % faster than without (2, 4 and 16 KiB:
-// 1.3-1.5 %); the forward's state buffers (block_views) measured no gain from
-// a pad.
+// pad the sweep on 2,097,152 triangles (Euler p = 4) ran 1.8 % faster than
+// without (2, 4 and 16 KiB: 1.3-1.5 %); the forward's state buffers
+// (block_views) measured no gain from a pad.
 struct AdjBuffers {
   std::vector<double *> bufs;
   void *block = nullptr;  // the group's own allocation, if it has one
@@ -1519,6 +1520,7 @@ struct AdjWorkspace {
   explicit AdjWorkspace(dg_handle *hh) : h(hh) {}
   AdjWorkspace(const AdjWorkspace &) = delete;
   ~AdjWorkspace() {
+    h->ws_busy = false;
     if (!h->d_ws) return;
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) != hipSuccess) (void)hipGetLastError();
@@ -1539,6 +1541,7 @@ struct AdjWorkspace {
       h->ws_bytes = bytes;
     }
     p = h->d_ws;
+    h->ws_busy = true;
     return DG_OK;
   }
   void take(AdjBuffers &ab, size_t count, size_t bytes) {

@@ -89,7 +89,6 @@ struct StageArgs {
   const double *un;  // step base    [N][NP][K]
   double *out;       // stage output
   double *acc;       // RK4 running combination
-  const double *u1, *u2;  // ACC_STAGES: the inputs of the second and third stage
   DevState *st;
   PhysParams ph;
   int mode, accmode;
@@ -127,6 +126,7 @@ struct StageArgs {
   // side points evaluate time-dependent boundary data
   int small, step_pos, conv_run, tdb;
   int *fired;  // set to 1 wherever the positivity fix fires or a stored state is flagged
+  const double *u1, *u2;  // ACC_STAGES: the inputs of the second and third stage
 };
 
 // doubles of stored traces per element: 3 sides x n_q1 points x 4 variables
