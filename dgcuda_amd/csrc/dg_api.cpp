@@ -709,11 +709,6 @@ static bool small_path(const dg_handle *h) {
   if (h->K > small_max_k(h->cfg.physics, h->cfg.p) || volume_mfma(h->cfg)) return false;
   return h->use_traces || !(h->cfg.physics == DG_EULER && h->cfg.p >= 4);
 }
-// ... and close each step inside the next one's first stage
-static bool small_fold(const dg_handle *h) {
-  return small_path(h) && small_blocks(h->cfg.p, h->K) <= kSmallFold;
-}
-
 static StageArgs base_args(dg_handle *h) {
   StageArgs a;
   std::memset(&a, 0, sizeof a);
@@ -750,6 +745,20 @@ static bool bnd_time_dependent(const dg_handle *h) {
           h->cfg.problem == DG_PROB_ADV_ROTHILL);
 }
 
+// Whether the stages evaluate moving boundary data themselves: the
+// point-parallel kernel, for the systems it has that form for.  Any system may
+// run a moving problem's boundary states; the others' are launched before each
+// stage, as everywhere else.
+static bool small_bnd(const dg_handle *h) {
+  return small_path(h) && small_moving_bnd(h->cfg.physics);
+}
+// ... and close each step inside the next one's first stage: not where a
+// launch before that stage reads the step's time and dt
+static bool small_fold(const dg_handle *h) {
+  return small_path(h) && small_blocks(h->cfg.p, h->K) <= kSmallFold &&
+         (small_bnd(h) || !bnd_time_dependent(h));
+}
+
 // whether d_bnd_val has to be formed for time t: not the caller's states, and
 // walls and fixed states once per mesh (the caller launches what forms it)
 static bool bnd_stale(dg_handle *h) {
@@ -766,10 +775,10 @@ static void refresh_bnd_fixed(dg_handle *h, double t) {
 
 // one stage launch, preceded by the boundary data at the stage time when needed
 static void launch_stage_bnd(dg_handle *h, const StageArgs &a) {
-  // (the point-parallel stage evaluates it where it is used)
   StageArgs s = a;
-  s.tdb = bnd_time_dependent(h) ? 1 : 0;
-  if (s.tdb && !s.small)
+  const bool moving = bnd_time_dependent(h);
+  s.tdb = moving && small_bnd(h) ? 1 : 0;
+  if (moving && !s.tdb)
     launch_bnd(h->cfg.physics, h->cfg.p, a.m, h->ph, h->d_st, a.cstage, 1, 0., h->stream);
   launch_stage(h->cfg.physics, h->cfg.p, s, h->stream);
 }

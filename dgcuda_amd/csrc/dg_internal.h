@@ -123,7 +123,7 @@ struct StageArgs {
   double *tr_out;
   // small meshes: the point-parallel stage (k_stage_s), its place in the
   // step, whether the run reduces the step-to-step change, and whether its
-  // side points evaluate time-dependent boundary data
+  // side points evaluate time-dependent boundary data (small_moving_bnd)
   int small, step_pos, conv_run, tdb;
   int *fired;  // set to 1 wherever the positivity fix fires or a stored state is flagged
   const double *u1, *u2;  // ACC_STAGES: the inputs of the second and third stage
@@ -204,6 +204,7 @@ int upload_tables(int p, const void *tab, size_t bytes);
 void launch_stage(int phys, int p, const StageArgs &a, hipStream_t s);
 int small_max_k(int phys, int p);      // largest mesh of the point-parallel stage
 int small_blocks(int p, int K);        // its blocks
+bool small_moving_bnd(int phys);       // whether it evaluates moving boundary data itself
 void launch_init(int phys, int p, const MeshDev &m, const PhysParams &ph, double *c, hipStream_t s);
 // per-element error integrals (norm 1 or 2), [N][K]
 void launch_err(int phys, int p, int norm, const MeshDev &m, const PhysParams &ph,

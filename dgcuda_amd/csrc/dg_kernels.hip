@@ -107,6 +107,12 @@ __global__ __launch_bounds__((stage_blk<PHYS, P>())) void k_stage(const StageArg
 
 int small_blocks(int p, int K) { return nblocks(K, small_eb(p)); }
 
+bool small_moving_bnd(int phys) {
+  bool r = false;
+  dispatch(phys, 0, [&](auto PH, auto) { r = small_tdb<decltype(PH)::value>(); });
+  return r;
+}
+
 // The point-parallel stage (dg_stage_s.h) up to these many elements.  Below,
 // the one-thread (or four-lane) stage costs the instruction stream of a
 // single wave whatever the mesh: us per SSP-RK3 stage, the step's close

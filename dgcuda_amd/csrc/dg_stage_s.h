@@ -133,8 +133,10 @@ __device__ __forceinline__ bool small_needs_fix(const PhysParams &ph,
   return s_bad[el] != 0;
 }
 
-// the problems whose outside states depend on time (the caller's boundary
-// states and every wall do not): only their systems have the TDB form
+// the systems whose stage has the TDB form (outside states that depend on
+// time, evaluated by the side points): those that the moving problems are
+// states of.  The others run a moving problem too, with a launch before the
+// stage (launch_stage_bnd).
 template <int PHYS>
 __host__ __device__ constexpr bool small_tdb() {
   return PHYS == PH_ADV || PHYS == PH_EULER;
