@@ -783,18 +783,30 @@ static void launch_stage_bnd(dg_handle *h, const StageArgs &a) {
   launch_stage(h->cfg.physics, h->cfg.p, s, h->stream);
 }
 
-// Whether a kernel on device dev can use the caller's array p in place: a
-// DG_DEVICE array in plain memory of that very device (a copy also takes
-// another device's or managed memory), aligned for doubles.
-static bool in_place(int dev, const void *p, int where) {
-  if (where != DG_DEVICE || ((uintptr_t)p & 7)) return false;
+// How the caller's array p of `bytes` is reached from a kernel on device dev.
+// IN_PLACE: a DG_DEVICE array in plain memory of that very device, aligned for
+// doubles.  TOO_SHORT: such an array, but its allocation ends before the array
+// does (a copy refuses it too; a kernel would not notice).  BY_COPY: the rest,
+// another device's or managed memory among them.
+enum Reach { TOO_SHORT = -1, BY_COPY = 0, IN_PLACE = 1 };
+static Reach reach(int dev, const void *p, int where, size_t bytes) {
+  if (where != DG_DEVICE || ((uintptr_t)p & 7)) return BY_COPY;
   hipPointerAttribute_t at;
+  void *base = nullptr;
+  size_t size = 0;
   if (hipPointerGetAttributes(&at, p) != hipSuccess) {
     (void)hipGetLastError();
-    return false;
+    return BY_COPY;
   }
-  return at.type == hipMemoryTypeDevice && !at.isManaged && at.device == dev;
+  if (at.type != hipMemoryTypeDevice || at.isManaged || at.device != dev) return BY_COPY;
+  if (hipMemGetAddressRange((hipDeviceptr_t *)&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
+    (void)hipGetLastError();
+    return BY_COPY;
+  }
+  const size_t off = (size_t)((const char *)p - (const char *)base);
+  return off <= size && bytes <= size - off ? IN_PLACE : TOO_SHORT;
 }
+static const char kShort[] = "%s: a device array ends before its %zu bytes";
 
 static bool overlap(const void *a, const void *b, size_t bytes) {
   return (const char *)a < (const char *)b + bytes && (const char *)b < (const char *)a + bytes;
@@ -829,7 +841,9 @@ extern "C" int dg_eval_rhs(dg_handle *h, const double *u, double t, double dt, d
   if (!h->K) return fail(h, DG_ERR_STATE, "dg_eval_rhs: no mesh");
   HIPCHK(h, hipSetDevice(h->cfg.device));
   const size_t sb = sizeof(double) * dofs(h);
-  if (in_place(h->cfg.device, u, where) && in_place(h->cfg.device, k, where) && !overlap(u, k, sb)) {
+  const Reach ru = reach(h->cfg.device, u, where, sb), rk = reach(h->cfg.device, k, where, sb);
+  if (ru == TOO_SHORT || rk == TOO_SHORT) return fail(h, DG_ERR_HIP, kShort, "dg_eval_rhs", sb);
+  if (ru == IN_PLACE && rk == IN_PLACE && !overlap(u, k, sb)) {
     rhs_launches(h, u, t, dt, k, h->d_st, h->d_bad, bnd_stale(h));
     HIPCHK(h, hipGetLastError());
   } else {
@@ -1679,8 +1693,12 @@ extern "C" int dg_adjoint_rhs(dg_handle *h, const double *u, double t, double dt
   const size_t sb = sizeof(double) * dofs(h);
   // in place as dg_eval_rhs, else through the handle's buffers (the output's
   // is made by the first such call and goes with the mesh)
-  const bool direct = in_place(h->cfg.device, u, where) && in_place(h->cfg.device, gk, where) && in_place(h->cfg.device, gu, where) &&
-                      !overlap(u, gu, sb) && !overlap(gk, gu, sb);
+  bool direct = !overlap(u, gu, sb) && !overlap(gk, gu, sb);
+  for (const double *x : {u, gk, (const double *)gu}) {
+    const Reach r = reach(h->cfg.device, x, where, sb);
+    if (r == TOO_SHORT) return fail(h, DG_ERR_HIP, kShort, "dg_adjoint_rhs", sb);
+    direct = direct && r == IN_PLACE;
+  }
   const double *ui = u, *gi = gk;
   double *go = gu;
   if (!direct) {
@@ -2596,7 +2614,10 @@ extern "C" int dg_ens_get_coeffs(dg_ensemble *E, int i, double *C, int where) {
   auto &G = E->grp[h->cfg.p];
   const size_t kd = sizeof(double) * h->K;
   EHIPCHK(E, hipSetDevice(E->cfg.device));
-  if (in_place(E->cfg.device, C, where)) {
+  const size_t bytes = kd * E->N * h->np;
+  const Reach r = reach(E->cfg.device, C, where, bytes);
+  if (r == TOO_SHORT) return efail(E, DG_ERR_HIP, kShort, "dg_ens_get_coeffs", bytes);
+  if (r == IN_PLACE) {
     // one launch for all rows: a copy each was a fifth of a 20-step run's time
     // on 16 instances (350 copies)
     launch_rows(E->N * h->np, h->K, C, h->K, G.c + E->inst_off[i], G.K, E->stream);
@@ -2624,7 +2645,10 @@ extern "C" int dg_ens_set_coeffs(dg_ensemble *E, int i, const double *C, int whe
   auto &G = E->grp[h->cfg.p];
   const size_t kd = sizeof(double) * h->K;
   EHIPCHK(E, hipSetDevice(E->cfg.device));
-  if (in_place(E->cfg.device, C, where)) {
+  const size_t bytes = kd * E->N * h->np;
+  const Reach r = reach(E->cfg.device, C, where, bytes);
+  if (r == TOO_SHORT) return efail(E, DG_ERR_HIP, kShort, "dg_ens_set_coeffs", bytes);
+  if (r == IN_PLACE) {
     launch_rows(E->N * h->np, h->K, G.c + E->inst_off[i], G.K, C, h->K, E->stream);
     EHIPCHK(E, hipGetLastError());
     EHIPCHK(E, hipStreamSynchronize(E->stream));
