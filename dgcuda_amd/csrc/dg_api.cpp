@@ -956,12 +956,6 @@ extern "C" int dg_eval_rhs_noalloc(dg_handle *h, const double *u, double t, doub
 
 // stage schedule of one fused step; io[s] is the input of stage s and
 // io[S] the step's output (io[0] is the step's base state); returns S
-// Without acc (single meshes of the systems without a positivity fix) RK4
-// keeps no running combination: its last stage forms the result from the stage
-// inputs io[1 .. 3], which then are three arrays.  A step moves 13 state-sized
-// arrays instead of 17 and no stage ends with a read-modify-write.  us per stage:
-// TE p = 3 on 199,712 triangles 63 / 55, p = 2 on 320,000 50.7 / 44.1, p = 5 on
-// 80,000 186 / 171; advection p = 1 on 500,000 21.2 / 18.5.
 static int make_stages(const StageArgs &a, int integrator, int pf, StageArgs *st,
                        double *const *io, double *acc, bool conv) {
   int n = 0;
@@ -986,15 +980,6 @@ static int make_stages(const StageArgs &a, int integrator, int pf, StageArgs *st
   };
   switch (integrator) {
     case DG_RK4:  // time_integrator.cu:244-393
-      if (!acc) {
-        push(M_US_CK, 0, 1, 0.5, ACC_NONE, 0.0);
-        push(M_UN_CK, 0, 0, 0.5, ACC_NONE, 0.5);
-        push(M_UN_CK, 0, 0, 1.0, ACC_NONE, 0.5);
-        push(M_KONLY, 0, 0, 0, ACC_STAGES, 1.0);
-        st[3].u1 = io[1];
-        st[3].u2 = io[2];
-        break;
-      }
       push(M_US_CK, 0, 1, 0.5, ACC_SET6, 0.0);
       push(M_UN_CK, 0, 0, 0.5, ACC_ADD3, 0.5);
       push(M_UN_CK, 0, 0, 1.0, ACC_ADD3, 0.5);
@@ -1033,11 +1018,6 @@ static int build_step_io(dg_handle *h, StageArgs *st, int cfl_mode, double *cons
       st[q].step_pos = q == 0 ? STEP_FIRST : (q == n - 1 ? STEP_LAST : STEP_MID);
   }
   return n;
-}
-
-// RK4's running combination (nullptr: from the stage states, make_stages)
-static double *rk4_acc(const dg_handle *h) {
-  return h->cfg.physics == DG_EULER || h->cfg.physics == DG_SWE ? h->d_acc : nullptr;
 }
 
 static int nstages_of(int integ) {
@@ -1079,9 +1059,7 @@ static int build_step(dg_handle *h, StageArgs *st, int cfl_mode, bool conv = fal
   io[0] = h->d_c;
   for (int s = 1; s < S; s++) io[s] = (s & 1) ? h->d_b1 : h->d_b2;
   io[S] = h->d_c;
-  double *const acc = rk4_acc(h);
-  if (S == 4 && !acc) io[3] = h->d_acc;
-  const int ns = build_step_io(h, st, cfl_mode, io, acc, conv);
+  const int ns = build_step_io(h, st, cfl_mode, io, h->d_acc, conv);
   // each stage reads its input's stored traces and stores its output's
   for (int q = 0; q < ns; q++) {
     st[q].tr_in = traces_of(h, io[q]);
@@ -1827,7 +1805,7 @@ extern "C" int dg_adjoint_solve(dg_handle *h, int nsteps, double dt, int every, 
       for (int r = 0; r < S; r++) io[r] = stb.bufs[(size_t)s * S + r];
       io[S] = stb.bufs[(size_t)(s + 1) * S];
       StageArgs st[4];
-      build_step_io(h, st, 0, io, rk4_acc(h));
+      build_step_io(h, st, 0, io, h->d_acc ? h->d_acc : h->d_b2);
       for (int r = 0; r < S; r++) {
         if (posfix_on(h)) {
           st[r].flags_in = 1;

@@ -54,9 +54,7 @@ struct DevState {
 };
 
 enum StageMode { M_KONLY = 0, M_US_CK = 1, M_A_UN_B_US_CK = 2, M_UN_CK = 3 };
-// ACC_STAGES: RK4's last stage from the stage states themselves (no positivity
-// fix has touched them): u + ((u1 - u) + 2 (u2 - u) + (u3 - u)) / 3 + k4 / 6
-enum AccMode { ACC_NONE = 0, ACC_SET6 = 1, ACC_ADD3 = 2, ACC_FINAL6 = 3, ACC_STAGES = 4 };
+enum AccMode { ACC_NONE = 0, ACC_SET6 = 1, ACC_ADD3 = 2, ACC_FINAL6 = 3 };
 
 // where a small-mesh stage stands in its step (k_stage_s); STEP_NONE: the
 // step is closed by a launch of its own (or there is none)
@@ -126,7 +124,6 @@ struct StageArgs {
   // side points evaluate time-dependent boundary data (small_moving_bnd)
   int small, step_pos, conv_run, tdb;
   int *fired;  // set to 1 wherever the positivity fix fires or a stored state is flagged
-  const double *u1, *u2;  // ACC_STAGES: the inputs of the second and third stage
 };
 
 // doubles of stored traces per element: 3 sides x n_q1 points x 4 variables

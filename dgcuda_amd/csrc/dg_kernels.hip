@@ -96,13 +96,13 @@ void launch_finish(DevState *st, const unsigned long long *part, int nblk, const
   hipLaunchKernelGGL(k_finish, dim3(1), dim3(BLK), 0, s, st, part, nblk, f);
 }
 
-template <int PHYS, int P, bool STAGES>
+template <int PHYS, int P>
 __global__ __launch_bounds__((stage_blk<PHYS, P>())) void k_stage(const StageArgs a) {
   constexpr int NP = np_of(P), NQ1 = P + 1, N = nvars_of(PHYS);
   constexpr int B = stage_blk<PHYS, P>();
   __shared__ double s_side[3 * NP * NQ1];
   __shared__ double s_c[N * NP][B];
-  stage_body<PHYS, P, B, false, STAGES>(a, blockIdx.x, a.nblk, s_side, s_c);
+  stage_body<PHYS, P, B>(a, blockIdx.x, a.nblk, s_side, s_c);
 }
 
 int small_blocks(int p, int K) { return nblocks(K, small_eb(p)); }
@@ -180,12 +180,7 @@ void launch_stage(int phys, int p, const StageArgs &a0, hipStream_t s) {
     } else {
       constexpr int B = stage_blk<ph, pp>();
       a.nblk = nblocks(a.m.K, B);
-      bool stages = false;
-      if constexpr (!has_positivity<ph>()) stages = a.accmode == ACC_STAGES;
-      if (stages)
-        hipLaunchKernelGGL((k_stage<ph, pp, !has_positivity<ph>()>), dim3(a.nblk), dim3(B), 0, s, a);
-      else
-        hipLaunchKernelGGL((k_stage<ph, pp, false>), dim3(a.nblk), dim3(B), 0, s, a);
+      hipLaunchKernelGGL((k_stage<ph, pp>), dim3(a.nblk), dim3(B), 0, s, a);
     }
   });
   if (a.last_stage && a.step_pos == STEP_NONE) {
@@ -220,7 +215,7 @@ int stage_vgprs(int phys, int p, bool vol_mfma) {
     else if constexpr (stage_quad<ph, pp>())
       fn = reinterpret_cast<const void *>(&k_stage_q<ph, pp, false, true>);
     else
-      fn = reinterpret_cast<const void *>(&k_stage<ph, pp, false>);
+      fn = reinterpret_cast<const void *>(&k_stage<ph, pp>);
     if (hipFuncGetAttributes(&attr, fn) == hipSuccess) v = attr.numRegs;
   });
   return v;

@@ -216,11 +216,6 @@ __device__ __forceinline__ void fix_read(const PhysParams &ph, bool flags, int f
   }
 }
 
-// ACC_STAGES (the differences of nearby values are exact)
-__device__ __forceinline__ double rk4_stages(double u, double u1, double u2, double u3, double k) {
-  return u + (((u1 - u) + 2. * (u2 - u) + (u3 - u)) * (1. / 3.) + k * (1. / 6.));
-}
-
 // One RK stage over all elements, one thread per element (see the header
 // comment).  The element's memory accesses are software-pipelined: its own
 // state, its three side slots and side 0's neighbour are requested at entry;
@@ -255,9 +250,7 @@ __host__ __device__ constexpr int stage_blk() {
 // the mesh is an ensemble's merged mesh and a.ens[block] gives
 // its instance (whose DevState it reads), the instance's first element and
 // its end; elements from the end to the block's end are padding.
-// STAGES: RK4's last stage from the stage states (ACC_STAGES), a kernel of its
-// own: beside the other combinations its loads cost the second wave per SIMD.
-template <int PHYS, int P, int B, bool ENS = false, bool STAGES = false>
+template <int PHYS, int P, int B, bool ENS = false>
 __device__ __forceinline__ void stage_body(const StageArgs a, int pblock, int nblk,
                                            double *s_side, double (*s_c)[B]) {
   using TC = TabC<P>;
@@ -288,7 +281,7 @@ __device__ __forceinline__ void stage_body(const StageArgs a, int pblock, int nb
   const int ee = act ? e : eend - 1;
   const double dt = st->dt;
   const bool flags = a.flags_in != 0;
-  const bool use_un = STAGES || a.accmode == ACC_FINAL6 || a.mode == M_A_UN_B_US_CK || a.mode == M_UN_CK;
+  const bool use_un = a.accmode == ACC_FINAL6 || a.mode == M_A_UN_B_US_CK || a.mode == M_UN_CK;
 
   // ---- requested at entry: the slots (first: loads complete in order, and
   // the neighbour index waits only for them), own state, side 0's neighbour
@@ -575,36 +568,11 @@ __device__ __forceinline__ void stage_body(const StageArgs a, int pblock, int nb
   // Shu-Osher forms); the branches are uniform.  The step base un was
   // requested during the last side.
   double (&o)[N][NP] = c;
-  double dc = 0.;
   if constexpr (!kPipe) {
-    if (!STAGES && use_un) load_state(a.un, K, ee, ub);
+    if (use_un) load_state(a.un, K, ee, ub);
   }
-  if (!STAGES && use_un && a.fix_un) fix_read<PHYS, P>(a.ph, flags, fl_me, ub);
-  if constexpr (STAGES) {
-    // a variable at a time, stored at once (and the input from its parked
-    // copy): all of them in flight do not fit the registers
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int n = 0; n < N; n++) {
-      double x[NP], y[NP], u[NP];
-#pragma unroll
-      for (int i = 0; i < NP; i++) {
-        u[i] = kPipe ? ub[n][i] : gld(a.un + (size_t)(n * NP + i) * K, ee);
-        x[i] = gld(a.u1 + (size_t)(n * NP + i) * K, ee);
-        y[i] = gld(a.u2 + (size_t)(n * NP + i) * K, ee);
-      }
-#pragma unroll
-      for (int i = 0; i < NP; i++) {
-        const double v = rk4_stages(u[i], x[i], y[i], s_c[n * NP + i][threadIdx.x], acc[n][i]);
-        if (a.conv && act && n * NP + i < N) dc = fmax(dc, fabs(v - u[i]));
-        if (act) gst_nt(a.out + (size_t)(n * NP + i) * K, e, v);
-        if (i == 0) o[n][0] = v;
-      }
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  } else if (a.accmode == ACC_FINAL6) {
+  if (use_un && a.fix_un) fix_read<PHYS, P>(a.ph, flags, fl_me, ub);
+  if (a.accmode == ACC_FINAL6) {
 #pragma unroll
     for (int n = 0; n < N; n++)
 #pragma unroll
@@ -670,12 +638,13 @@ __device__ __forceinline__ void stage_body(const StageArgs a, int pblock, int nb
   // step-to-step change before the store (out may alias un)
   // (the reference's norm covers the first K*N state entries: rows
   // n * n_p + i < N, time_integrator.cu:404-414)
-  if (!STAGES && a.conv && act) {
+  double dc = 0.;
+  if (a.conv && act) {
 #pragma unroll
     for (int r = 0; r < N && r < N * NP; r++)
       dc = fmax(dc, fabs(o[r / NP][r % NP] - gld(a.un + (size_t)r * K, ee)));
   }
-  if (!STAGES && act) {
+  if (act) {
 #pragma unroll
     for (int n = 0; n < N; n++)
 #pragma unroll

@@ -170,10 +170,10 @@ __global__ __launch_bounds__((small_t<PHYS, P, FULL>())) void k_stage_s(const St
   const int e = remap_block(blockIdx.x, a.nblk) * EB + el;
   const bool act = e < K;
   const int ee = act ? e : K - 1;
-  const bool use_un = a.accmode >= ACC_FINAL6 || a.mode == M_A_UN_B_US_CK || a.mode == M_UN_CK;
+  const bool use_un = a.accmode == ACC_FINAL6 || a.mode == M_A_UN_B_US_CK || a.mode == M_UN_CK;
 
   // ---- every load that needs no other goes out first
-  double own[R], ub[R], ra[R], rb[R];
+  double own[R], ub[R], ra[R];
 #pragma unroll
   for (int q = 0; q < R; q++) {
     const int r = row + q * RW, rr = r < NR ? r : 0;
@@ -206,13 +206,9 @@ __global__ __launch_bounds__((small_t<PHYS, P, FULL>())) void k_stage_s(const St
 #pragma unroll
   for (int q = 0; q < R; q++) {
     const int r = row + q * RW, rr = r < NR ? r : 0;
-    ub[q] = ra[q] = rb[q] = 0.;
+    ub[q] = ra[q] = 0.;
     if (use_un || a.conv) ub[q] = gld(a.un + (size_t)rr * K, ee);
     if (a.accmode == ACC_ADD3 || a.accmode == ACC_FINAL6) ra[q] = gld(a.acc + (size_t)rr * K, ee);
-    if (!has_positivity<PHYS>() && a.accmode == ACC_STAGES) {
-      ra[q] = gld(a.u1 + (size_t)rr * K, ee);
-      rb[q] = gld(a.u2 + (size_t)rr * K, ee);
-    }
   }
   // the step state; the first stage of a step closes the step before it
   DevState S = a.st[(a.step_pos == STEP_MID || a.step_pos == STEP_LAST) ? 1 : 0];
@@ -440,8 +436,6 @@ __global__ __launch_bounds__((small_t<PHYS, P, FULL>())) void k_stage_s(const St
     }
     if (a.accmode == ACC_FINAL6) {
       o[q] = un + (ra[q] + acc * (1. / 6.));
-    } else if (!has_positivity<PHYS>() && a.accmode == ACC_STAGES) {
-      o[q] = rk4_stages(un, ra[q], rb[q], us, acc);
     } else {
       if (a.accmode == ACC_SET6 && mine) gst(a.acc + (size_t)r * K, e, acc * (1. / 6.));
       if (a.accmode == ACC_ADD3 && mine) gst(a.acc + (size_t)r * K, e, ra[q] + acc * (1. / 3.));
