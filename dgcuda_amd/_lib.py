@@ -36,7 +36,7 @@ EXPORTS = [
     "dg_load_pmsh", "dg_set_eps", "dg_project_ic", "dg_set_coeffs", "dg_get_coeffs",
     "dg_eval_rhs", "dg_eval_rhs_noalloc", "dg_step", "dg_run", "dg_l2_error", "dg_l1_error", "dg_eval_exact", "dg_eval_u", "dg_lambda", "dg_limit", "dg_info",
     "dg_geometry", "dg_sync", "dg_stream", "dg_last_timing", "dg_adjoint_set_objective",
-    "dg_adjoint_solve", "dg_adjoint_rhs", "dg_adjoint_timing", "dg_adjoint_objective",
+    "dg_adjoint_solve", "dg_adjoint_release", "dg_adjoint_rhs", "dg_adjoint_timing", "dg_adjoint_objective",
     "dg_ens_create", "dg_ens_destroy", "dg_ens_last_error", "dg_ens_add", "dg_ens_build",
     "dg_ens_step", "dg_ens_get_coeffs", "dg_ens_set_coeffs", "dg_ens_state", "dg_ens_info",
     "dg_ens_l2_error", "dg_boundary_points", "dg_set_boundary_states", "dg_get_boundary_states",
@@ -115,6 +115,7 @@ def load():
         "dg_last_timing": (I, [H, P(D), P(I)]),
         "dg_adjoint_set_objective": (I, [H, I, VP, I, VP, I]),
         "dg_adjoint_solve": (I, [H, I, D, I, P(D), VP, VP, I]),
+        "dg_adjoint_release": (I, [H]),
         "dg_adjoint_rhs": (I, [H, VP, D, D, VP, VP, I]),
         "dg_adjoint_timing": (I, [H, P(D), P(D)]),
         "dg_adjoint_objective": (I, [H, P(D)]),

@@ -18,12 +18,14 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
 #include "../../include/dg.h"
 #include "dg_internal.h"
 #include "dg_ref_tables.h"
+#include "dg_workspace.h"
 
 using namespace dgk;
 
@@ -70,11 +72,7 @@ struct dg_handle {
   double *d_err = nullptr, *d_lam = nullptr;
   DevState *d_st = nullptr;  // [2]: the state between steps, the running step's (k_stage_s)
   unsigned long long *d_part = nullptr;  // per-block maxima of the step reduction
-  char *d_ws = nullptr;                  // dg_adjoint_solve's buffers, kept for the next call
-  size_t ws_bytes = 0;
-  bool ws_busy = false;                  // a solve is using them
   double *d_red = nullptr;               // [kSumBlocks + 1] objective sum: partials, result
-  double *d_gu = nullptr;                // dg_adjoint_rhs's output before its copy out
   int *d_bad = nullptr;                  // positivity flags of the stored state d_c
   // graphs of 2^q steps, q < kGraphLevels (same configuration key)
   hipGraphExec_t graph[kGraphLevels] = {};
@@ -114,19 +112,29 @@ static int fail(dg_handle *h, int code, const char *fmt, ...) {
       return fail(h, DG_ERR_HIP, "%s failed: %s", #x, hipGetErrorString(e_));         \
   } while (0)
 
+// the adjoint buffers that handles keep (never destroyed: handles may outlive
+// the process's static objects)
+static void kept_free(void *p) { (void)hipFree(p); }
+static KeptBuffers<kept_free> &kept() {
+  static auto *k = new KeptBuffers<kept_free>();
+  return *k;
+}
+
+// every allocation of the library on device dev (an error is the caller's to
+// report: the next call's launch check does not see it)
+static hipError_t dev_malloc(int dev, void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && kept().reclaim(dev)) e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
 static int alloc(dg_handle *h, void **p, size_t bytes) {
   if (*p) {
     (void)hipFree(*p);
     *p = nullptr;
   }
-  hipError_t e = hipMalloc(p, bytes ? bytes : 8);
-  if (e != hipSuccess && h->d_ws && !h->ws_busy) {  // the kept adjoint buffers go first
-    (void)hipGetLastError();
-    (void)hipFree(h->d_ws);
-    h->d_ws = nullptr;
-    h->ws_bytes = 0;
-    e = hipMalloc(p, bytes ? bytes : 8);
-  }
+  hipError_t e = dev_malloc(h->cfg.device, p, bytes ? bytes : 8);
   if (e != hipSuccess)
     return fail(h, DG_ERR_HIP, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
   return DG_OK;
@@ -341,7 +349,7 @@ extern "C" int dg_create(dg_handle **out, const dg_config *cfg) {
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreate(&h->ev0) != hipSuccess || hipEventCreate(&h->ev1) != hipSuccess ||
       ensure_tables(cfg->device, cfg->p) != 0 || ensure_scratch(cfg->device) != 0 ||
-      hipMalloc((void **)&h->d_st, 2 * sizeof(DevState)) != hipSuccess) {
+      dev_malloc(cfg->device, (void **)&h->d_st, 2 * sizeof(DevState)) != hipSuccess) {
     dg_destroy(h);
     return DG_ERR_HIP;
   }
@@ -370,9 +378,8 @@ static void free_mesh(dg_handle *h) {
   dfree(h->d_trblk);
   for (auto &t : h->d_tr) t = nullptr;
   for (auto &k : h->d_k) dfree(k);
-  dfree(h->d_err); dfree(h->d_lam); dfree(h->d_gw); dfree(h->d_gu);
-  dfree(h->d_ws); dfree(h->d_red);
-  h->ws_bytes = 0; dfree(h->d_part); dfree(h->d_bad);
+  dfree(h->d_err); dfree(h->d_lam); dfree(h->d_gw); dfree(h->d_red); dfree(h->d_part); dfree(h->d_bad);
+  kept().drop(h);
   drop_graphs(h);
   // no mesh from here until a new one is fully uploaded: every call that
   // needs one checks K, and the objective's weights went with the buffers
@@ -1316,7 +1323,7 @@ extern "C" int dg_eval_exact(dg_handle *h, int n, double t, double *u1, double *
   if (n >= h->N) return fail(h, DG_ERR_ARG, "dg_eval_exact: variable %d of %d", n, h->N);
   HIPCHK(h, hipSetDevice(h->cfg.device));
   double *d = nullptr;
-  HIPCHK(h, hipMalloc((void **)&d, sizeof(double) * 3 * h->K));
+  HIPCHK(h, dev_malloc(h->cfg.device, (void **)&d, sizeof(double) * 3 * h->K));
   launch_exact_vertex(h->cfg.physics, mesh_dev(h), h->ph, t, n, d, d + h->K, d + 2 * h->K,
                       h->stream);
   hipError_t e = hipGetLastError();
@@ -1340,7 +1347,7 @@ extern "C" int dg_eval_u(dg_handle *h, int n, double *u1, double *u2, double *u3
   double *o1 = h->d_lam, *o2 = d, *o3 = d + h->K;
   double *extra = nullptr;
   if (h->N < 2) {
-    HIPCHK(h, hipMalloc((void **)&extra, sizeof(double) * 2 * h->K));
+    HIPCHK(h, dev_malloc(h->cfg.device, (void **)&extra, sizeof(double) * 2 * h->K));
     o2 = extra;
     o3 = extra + h->K;
   }
@@ -1500,7 +1507,7 @@ static void adj_views(AdjBuffers &ab, char *base, size_t count, size_t bytes) {
 static int adj_alloc(dg_handle *h, AdjBuffers &ab, size_t count, size_t bytes) {
   if (!count) return DG_OK;
   void *p = nullptr;
-  hipError_t e = hipMalloc(&p, adj_stride(bytes) * count);
+  hipError_t e = dev_malloc(h->cfg.device, &p, adj_stride(bytes) * count);
   if (e != hipSuccess)
     return fail(h, DG_ERR_HIP, "adjoint: hipMalloc of %zu buffers of %zu bytes failed (%s)", count,
                 bytes, hipGetErrorString(e));
@@ -1509,40 +1516,40 @@ static int adj_alloc(dg_handle *h, AdjBuffers &ab, size_t count, size_t bytes) {
   return DG_OK;
 }
 
-// The work buffers of a solve lie in one allocation that the handle keeps for
-// the next solve, up to 1/32 of the device's memory (9 GB): allocating and
-// freeing them was 1.7 ms of a 33 ms gradient (TE p = 3, 199,712 triangles, 32
-// steps, 5.6 GB) and 1.0 of 10.4 (Euler p = 4, 131,072, 8 steps).  Larger ones
-// are given back at once; the rest with the mesh, or when an allocation fails.
+// The work buffers of a solve lie in one allocation.  A solve that has ended
+// leaves it to the handle's next one (dg_workspace.h) up to 1/32 of the device's
+// memory (9 GB) for all handles together; a call that fails frees it.
 struct AdjWorkspace {
   dg_handle *h;
   char *p = nullptr;
-  size_t used = 0;
+  size_t bytes = 0, used = 0;
+  bool ended = false;  // the stream has been waited for: nothing uses the buffers
   explicit AdjWorkspace(dg_handle *hh) : h(hh) {}
   AdjWorkspace(const AdjWorkspace &) = delete;
   ~AdjWorkspace() {
-    h->ws_busy = false;
-    if (!h->d_ws) return;
+    if (!p) return;
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) != hipSuccess) (void)hipGetLastError();
-    if (h->ws_bytes <= tot / 32) return;
-    dfree(h->d_ws);
-    h->ws_bytes = 0;
-  }
-  int reserve(size_t bytes) {
-    if (h->ws_bytes < bytes) {
-      dfree(h->d_ws);
-      h->ws_bytes = 0;
-      const hipError_t e = hipMalloc((void **)&h->d_ws, bytes);
-      if (e != hipSuccess) {
-        h->d_ws = nullptr;
-        return fail(h, DG_ERR_HIP, "adjoint: hipMalloc of %zu bytes failed (%s)", bytes,
-                    hipGetErrorString(e));
+    try {
+      if (ended) {
+        kept().give(h, h->cfg.device, p, bytes, tot / 32);
+        return;
       }
-      h->ws_bytes = bytes;
+    } catch (const std::bad_alloc &) {  // (no room for the note of it)
     }
-    p = h->d_ws;
-    h->ws_busy = true;
+    (void)hipFree(p);
+  }
+  int reserve(size_t need) {
+    p = (char *)kept().take(h, &bytes);
+    if (bytes >= need) return DG_OK;
+    dfree(p);
+    const hipError_t e = dev_malloc(h->cfg.device, (void **)&p, need);
+    if (e != hipSuccess) {
+      p = nullptr;
+      return fail(h, DG_ERR_HIP, "adjoint: hipMalloc of %zu bytes failed (%s)", need,
+                  hipGetErrorString(e));
+    }
+    bytes = need;
     return DG_OK;
   }
   void take(AdjBuffers &ab, size_t count, size_t bytes) {
@@ -1669,8 +1676,8 @@ extern "C" int dg_adjoint_rhs(dg_handle *h, const double *u, double t, double dt
                 "adjoint: the limiter is not differentiated");
   HIPCHK(h, hipSetDevice(h->cfg.device));
   const size_t sb = sizeof(double) * dofs(h);
-  // in place as dg_eval_rhs, else through the handle's buffers (the output's
-  // is made by the first such call and goes with the mesh)
+  // in place as dg_eval_rhs, else through the handle's buffers and one for the
+  // output
   bool direct = !overlap(u, gu, sb) && !overlap(gk, gu, sb);
   for (const double *x : {u, gk, (const double *)gu}) {
     const Reach r = reach(h->cfg.device, x, where, sb);
@@ -1679,16 +1686,15 @@ extern "C" int dg_adjoint_rhs(dg_handle *h, const double *u, double t, double dt
   }
   const double *ui = u, *gi = gk;
   double *go = gu;
+  AdjBuffers ab;
   if (!direct) {
-    if (!h->d_gu) {
-      const int rc = alloc(h, (void **)&h->d_gu, sb);
-      if (rc) return rc;
-    }
+    const int rc = adj_alloc(h, ab, 1, sb);
+    if (rc) return rc;
     HIPCHK(h, hipMemcpyAsync(h->d_b1, u, sb, kind_to(where), h->stream));
     HIPCHK(h, hipMemcpyAsync(h->d_b2, gk, sb, kind_to(where), h->stream));
     ui = h->d_b1;
     gi = h->d_b2;
-    go = h->d_gu;
+    go = ab.bufs[0];
   }
   refresh_bnd_fixed(h, t);
   launch_adjoint_rhs(h->cfg.physics, h->cfg.p, adj_args(h, ui, gi, go, nullptr, dt), h->stream);
@@ -1967,6 +1973,14 @@ extern "C" int dg_adjoint_solve(dg_handle *h, int nsteps, double dt, int every, 
     HIPCHK(h, hipMemcpyAsync(&fired, h->d_fired, sizeof(int), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
   h->adj_fix_fired = fired ? 1 : 0;
+  ws.ended = true;
+  return DG_OK;
+}
+
+extern "C" int dg_adjoint_release(dg_handle *h) {
+  if (!h) return DG_ERR_ARG;
+  HIPCHK(h, hipSetDevice(h->cfg.device));
+  kept().drop(h);
   return DG_OK;
 }
 
@@ -2075,7 +2089,7 @@ static int efail(dg_ensemble *E, int code, const char *fmt, ...) {
 template <typename T>
 static int ealloc(dg_ensemble *E, T *&p, size_t count) {
   dfree(p);
-  hipError_t e = hipMalloc((void **)&p, sizeof(T) * (count ? count : 1));
+  hipError_t e = dev_malloc(E->cfg.device, (void **)&p, sizeof(T) * (count ? count : 1));
   if (e != hipSuccess)
     return efail(E, DG_ERR_HIP, "hipMalloc(%zu) failed: %s", sizeof(T) * count,
                  hipGetErrorString(e));

@@ -273,6 +273,11 @@ class Solver:
                           RuntimeWarning, stacklevel=2)
         return J.value, gu, ge
 
+    def adjoint_release(self):
+        """frees the device buffers that adjoint_solve has left for the next
+        solve (before another library's large allocation, for instance)"""
+        self._chk(self.lib.dg_adjoint_release(self.h))
+
     def adjoint_rhs(self, u, gk, t=0.0, dt=1.0):
         """(dk/du)^T gk for k = dt * L(u); CUDA tensors in give a CUDA tensor
         out (no host copy), host data a numpy array"""
