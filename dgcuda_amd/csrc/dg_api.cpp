@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "../../include/dg.h"
+#include "dg_adj_plan.h"
 #include "dg_internal.h"
 #include "dg_ref_tables.h"
 #include "dg_workspace.h"
@@ -1497,8 +1498,6 @@ struct AdjBuffers {
   }
 };
 
-static size_t adj_stride(size_t bytes) { return (bytes + 255) / 256 * 256 + 8192; }
-
 static void adj_views(AdjBuffers &ab, char *base, size_t count, size_t bytes) {
   for (size_t q = 0; q < count; q++) ab.bufs.push_back((double *)(base + q * adj_stride(bytes)));
 }
@@ -1561,15 +1560,13 @@ struct AdjWorkspace {
 // How many of a checkpointed solve's segments keep the stage data of the
 // forward pass itself (the last ones), so that the reverse sweep walks them
 // without recomputing.  Off unless DG_ADJ_STORE_GB gives a memory budget in
-// GB: then as many as it and the free device memory hold, less a margin (5 %
-// of the device or 2 GiB, whichever is more), after the checkpoints and the
-// recompute buffers that the other segments need.  (Off by default: fresh
+// GB: then as many as it and the device memory hold, free or in idle kept
+// buffers (which an allocation takes when it has to), less a margin: 5 % of the
+// device or 2 GiB, whichever is more.  (Off by default: fresh
 // allocations of that size cost more than the recompute they save, e.g.
-// 271 GB for 54 of config 4's 125 segments took 2.2 s to allocate and free
-// against 0.23 s of recompute saved.)  seg_bytes(ns) is one segment's stage
-// data for ns steps.
-template <class F>
-static int resident_segments(int nsteps, int every, int nseg, size_t sb, const F &seg_bytes) {
+// 271 GB for 54 of the 125 segments of 2,000 steps on 199,712 triangles took
+// 2.2 s to allocate and free against 0.23 s of recompute saved.)
+static int resident_segments(const dg_handle *h, const AdjPlan &plan) {
   const char *env = std::getenv("DG_ADJ_STORE_GB");
   if (!env) return 0;
   char *end = nullptr;
@@ -1580,25 +1577,9 @@ static int resident_segments(int nsteps, int every, int nseg, size_t sb, const F
     (void)hipGetLastError();
     return 0;
   }
+  const size_t avail = fr + kept().idle(h->cfg.device);
   const size_t margin = std::max(tot / 20, (size_t)2 << 30);
-  size_t budget = fr > margin ? fr - margin : 0;
-  const double cap = gb * 1e9;  // compared as a double: no overflow for a large setting
-  if (cap < (double)budget) budget = (size_t)cap;
-  auto len = [&](int q) { return std::min(every, nsteps - q * every); };
-  size_t all = 0;
-  for (int q = 0; q < nseg; q++) all += seg_bytes(len(q));
-  if (all <= budget) return nseg;  // no checkpoints, no recompute
-  // segment 0 at least is recomputed: the recompute buffers and a checkpoint
-  // per recomputed segment; each resident segment saves its checkpoint
-  size_t used = seg_bytes(every) + (size_t)nseg * sb;
-  int r = 0;
-  for (int q = nseg - 1; q > 0; q--) {
-    const size_t add = seg_bytes(len(q)) - sb;
-    if (used + add > budget) break;
-    used += add;
-    r++;
-  }
-  return r;
+  return plan.resident(gb * 1e9, avail > margin ? avail - margin : 0);
 }
 
 extern "C" int dg_adjoint_set_objective(dg_handle *h, int kind, const double *params, int nparams,
@@ -1729,22 +1710,16 @@ extern "C" int dg_adjoint_solve(dg_handle *h, int nsteps, double dt, int every, 
   AdjBuffers ck, store, kst, wk;
   int rc;
   if (traces_wanted(h) && (rc = alloc_traces(h)) != DG_OK) return rc;
-  const int nres = resident_segments(nsteps, every, nseg, sb, [&](int ns) {
-    return ((size_t)ns * S + 1) * sb + (want_eps ? (size_t)ns * S * kst_b : 0);
-  });
+  AdjPlan plan{nsteps, every, S, sb, 0, 0};
+  if (want_eps) {
+    plan.kst_b = kst_b;
+    plan.eps_b = adj_stride(sizeof(double) * h->K) + adj_stride(2 * sizeof(double) * h->S);
+  }
+  const int nres = resident_segments(h, plan), nrec = plan.nrec(nres);
   h->adj_resident = nres;
-  // Segments 0 .. nrec - 1 are recomputed.  The last one never is: the sweep
-  // starts there, so its forward pass leaves its stage data in the recompute's
-  // buffers (unless it is resident anyway).
-  const int nrec = nres ? nseg - nres : nseg - 1;
   const size_t seg_stages = nres < nseg ? (size_t)every * S : 0;
-  size_t need = adj_stride(sb) * (S + 2 + nrec);
-  if (nres < nseg) need += adj_stride(sb) * (seg_stages + 1);
-  if (want_eps)
-    need += adj_stride(kst_b) * seg_stages + adj_stride(sizeof(double) * h->K) +
-            adj_stride(2 * sizeof(double) * h->S);
   AdjWorkspace ws(h);
-  if ((rc = ws.reserve(need)) != DG_OK) return rc;
+  if ((rc = ws.reserve(plan.need(nres))) != DG_OK) return rc;
   ws.take(wk, S + 2, sb);
   ws.take(ck, nrec, sb);
   if (nres < nseg) {

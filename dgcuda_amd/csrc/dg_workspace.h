@@ -94,6 +94,14 @@ class KeptBuffers {
     }
     for (void *q : out) FREE(q);
   }
+  // bytes of the device in idle buffers
+  size_t idle(int device) {
+    std::lock_guard<std::mutex> l(m);
+    size_t sum = 0;
+    for (const Kept &k : v)
+      if (k.device == device) sum += k.bytes;
+    return sum;
+  }
   void drop(const void *owner) {
     release([&](const Kept &k) { return k.owner == owner; });
   }

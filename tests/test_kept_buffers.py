@@ -31,13 +31,13 @@ int main() {
   K.give(&h[0], 0, a, 40, 100);
   K.give(&h[1], 0, b, 50, 100);
   K.give(&h[2], 1, c, 100, 100);          // another device: its own bound
-  CHECK(live == 4);
+  CHECK(live == 4 && K.idle(0) == 90 && K.idle(1) == 100 && K.idle(2) == 0);
   K.give(&h[3], 0, d, 60, 100);           // 150: the oldest goes, then the next
   CHECK(a->state == 2 && b->state == 2 && c->state == 0 && live == 2);
   CHECK(K.take(&h[0], &n) == nullptr && K.take(&h[3], &n) == d && n == 60);
   K.give(&h[3], 0, d, 101, 100);          // larger than the bound: not kept
   CHECK(d->state == 2 && K.take(&h[3], &n) == nullptr && live == 1);
-  CHECK(!K.reclaim(0) && K.reclaim(1) && c->state == 2 && !K.reclaim(1) && live == 0);
+  CHECK(K.idle(0) == 0 && !K.reclaim(0) && K.reclaim(1) && c->state == 2 && !K.reclaim(1) && live == 0);
   a = fresh(); b = fresh();
   K.give(&h[0], 0, a, 10, 100);
   K.give(&h[1], 0, b, 10, 100);
