@@ -99,8 +99,10 @@ class Solver:
         return out.ctypes.data, _lib.HOST
 
     def _wait(self, t):
-        """what torch has queued on its current stream (the tensor's values,
-        readers of an output): the solver's stream does not wait for it"""
+        """waits for what torch has queued on its current stream, which the
+        solver's stream does not: an input's values, readers of the memory that
+        an output is written to (a new tensor's may be a freed one's).  Calls
+        with inputs and outputs wait once, for the input."""
         cuda = _torch().cuda
         if not cuda.is_current_stream_capturing():
             cuda.current_stream(t.device).synchronize()
@@ -193,6 +195,8 @@ class Solver:
         if out is None:
             out = np.empty(self.shape)
         a, where = self._out(out, self.size, "coeffs")
+        if where == _lib.DEVICE:
+            self._wait(out)
         self._chk(self.lib.dg_get_coeffs(self.h, a, where))
         return out
 
@@ -265,6 +269,8 @@ class Solver:
             ge = np.empty(self.K) if want_eps else None
         ga, where = self._out(gu, self.size, "grad_u0")
         ea = self._out(ge, self.K, "grad_eps")[0] if want_eps else None
+        if where == _lib.DEVICE:
+            self._wait(gu)
         self._chk(self.lib.dg_adjoint_solve(self.h, int(nsteps), float(dt), int(every),
                                             ctypes.byref(J), ga, ea, where))
         if self.info().adj_fix_fired:
