@@ -1398,7 +1398,9 @@ extern "C" int dg_info(dg_handle *h, dg_info_t *info) {
   info->dofs = (long long)dofs(h);
   info->min_r = h->min_r;
   (void)hipSetDevice(h->cfg.device);
-  info->vgprs_stage = stage_vgprs(h->cfg.physics, h->cfg.p, volume_mfma(h->cfg));
+  info->vgprs_stage = stage_vgprs(h->cfg.physics, h->cfg.p, volume_mfma(h->cfg),
+                                  h->K && small_path(h) ? small_blocks(h->cfg.p, h->K) : 0,
+                                  bnd_time_dependent(h));
   info->adj_fix_fired = h->adj_fix_fired;
   info->adj_resident = h->adj_resident;
   return DG_OK;

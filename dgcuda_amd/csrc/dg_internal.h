@@ -229,7 +229,7 @@ void launch_eval_u(int phys, int p, int K, const double *c, int n, double *u1, d
 // boundary data of every boundary slot at the stage time (or a fixed time)
 void launch_bnd(int phys, int p, const MeshDev &m, const PhysParams &ph, const DevState *st,
                 double cstage, int use_state, double t, hipStream_t s);
-int stage_vgprs(int phys, int p, bool vol_mfma);
+int stage_vgprs(int phys, int p, bool vol_mfma, int small_nblk, bool tdb);
 void launch_traces(int phys, int p, int K, const double *u, double *tr, hipStream_t s);
 
 // adjoint launchers (dg_adjoint.hip)

@@ -203,13 +203,27 @@ void launch_traces(int phys, int p, int K, const double *u, double *tr, hipStrea
   });
 }
 
-int stage_vgprs(int phys, int p, bool vol_mfma) {
+// registers of the kernel that launch_stage runs (small_nblk: the blocks of the
+// point-parallel one, 0 for the others)
+int stage_vgprs(int phys, int p, bool vol_mfma, int small_nblk, bool tdb) {
   int v = -1;
   dispatch(phys, p, [&](auto PH, auto PP) {
     constexpr int ph = decltype(PH)::value, pp = decltype(PP)::value;
     hipFuncAttributes attr;
     const void *fn;
-    if constexpr (volume_mfma_ok<ph, pp>())
+    if (small_nblk) {
+      auto pick = [&](auto FULL) {
+        constexpr bool full = decltype(FULL)::value;
+        fn = reinterpret_cast<const void *>(&k_stage_s<ph, pp, false, full>);
+        if constexpr (small_tdb<ph>()) {
+          if (tdb) fn = reinterpret_cast<const void *>(&k_stage_s<ph, pp, true, full>);
+        }
+      };
+      pick(std::true_type{});
+      if constexpr (!small_full(pp, 1 << 30)) {
+        if (!small_full(pp, small_nblk)) pick(std::false_type{});
+      }
+    } else if constexpr (volume_mfma_ok<ph, pp>())
       fn = vol_mfma ? reinterpret_cast<const void *>(&k_stage_q<ph, pp, true, true>)
                     : reinterpret_cast<const void *>(&k_stage_q<ph, pp, false, true>);
     else if constexpr (stage_quad<ph, pp>())
