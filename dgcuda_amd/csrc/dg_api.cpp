@@ -1443,8 +1443,10 @@ extern "C" int dg_last_timing(dg_handle *h, double *ms, int *stages) {
 //   gk_s = b_s g + sum_{r>s} a_rs l_r,  l_s = (dk/du(u_s))^T gk_s,
 //   adjoint of u^n = g + sum_s l_s.
 // Checkpoints of u^n are kept every `every` steps; the reverse sweep re-runs
-// each segment forward from its checkpoint (same fused stage kernels)
-// keeping every stage input, then walks the segment backwards.
+// a segment forward from its checkpoint (same fused stage kernels) keeping
+// every stage input, then walks the segment backwards.  The last segment is
+// not re-run: its forward pass keeps its stage inputs.  SSP-RK3 is transposed
+// in the form its stages run in, which writes one array per launch.
 
 namespace {
 struct Butcher {

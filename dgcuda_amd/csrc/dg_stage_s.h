@@ -15,8 +15,8 @@
 // The tables are in LDS, so the code is a few kilobytes.  The same launch
 // also does what the large-mesh path leaves to launches of their own: the
 // first stage of a step closes the step before it (every block reduces the
-// partials, block 0 stores the new step state), and time-dependent boundary
-// data are evaluated by the side points that use them.
+// partials, block 0 stores the new step state), and for advection and Euler
+// time-dependent boundary data are evaluated by the side points that use them.
 // Bound by latency: of 8.4 us per stage (supersonic vortex p = 3 on 2,880
 // triangles; 22.9 on the one-thread kernel with its boundary and close) 2.4 are
 // the launch, 2.6 the two dependent memory round trips and the store, the rest

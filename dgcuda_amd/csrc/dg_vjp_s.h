@@ -1,8 +1,8 @@
 // dg_vjp_s.h -- the right-hand side's vector-Jacobian product on small
 // meshes: a thread per point, then a thread per coefficient, as the small
-// mesh stage (dg_stage_s.h).  One launch does what the wide path does in up
-// two: for Maxwell TE's permittivity gradient the side points also form the
-// impedance terms (k_eps_side).
+// mesh stage (dg_stage_s.h).  For Maxwell TE's permittivity gradient, whose
+// impedance terms are a launch of their own on the wide path (k_eps_side), the
+// side points form those terms too.
 // Included by dg_adjoint.hip (the flux VJPs it uses are defined there).
 #pragma once
 
