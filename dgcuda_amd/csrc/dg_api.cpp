@@ -113,7 +113,7 @@ static int fail(dg_handle *h, int code, const char *fmt, ...) {
       return fail(h, DG_ERR_HIP, "%s failed: %s", #x, hipGetErrorString(e_));         \
   } while (0)
 
-// the adjoint buffers that handles keep (never destroyed: handles may outlive
+// the adjoint buffers that are kept (never destroyed: handles may outlive
 // the process's static objects)
 static void kept_free(void *p) { (void)hipFree(p); }
 static KeptBuffers<kept_free> &kept() {
@@ -1520,7 +1520,7 @@ static int adj_alloc(dg_handle *h, AdjBuffers &ab, size_t count, size_t bytes) {
 }
 
 // The work buffers of a solve lie in one allocation.  A solve that has ended
-// leaves it to the handle's next one (dg_workspace.h) up to 1/32 of the device's
+// leaves it to the device's next one (dg_workspace.h) up to 1/32 of the device's
 // memory (9 GB) for all handles together; a call that fails frees it.
 struct AdjWorkspace {
   dg_handle *h;
@@ -1543,9 +1543,9 @@ struct AdjWorkspace {
     (void)hipFree(p);
   }
   int reserve(size_t need) {
-    p = (char *)kept().take(h, &bytes);
-    if (bytes >= need) return DG_OK;
-    dfree(p);
+    p = (char *)kept().take(h, h->cfg.device, need, &bytes);
+    if (p) return DG_OK;
+    kept().drop(h);  // (too small)
     const hipError_t e = dev_malloc(h->cfg.device, (void **)&p, need);
     if (e != hipSuccess) {
       p = nullptr;

@@ -1,18 +1,19 @@
-// dg_workspace.h -- device buffers that handles keep between adjoint solves.
+// dg_workspace.h -- device buffers that are kept between adjoint solves.
 //
 // A solve's work buffers are gigabytes that live for milliseconds: allocating
 // and freeing 1 GB took 1 to 28 ms beside 8 ms of gradient (Euler p = 4, 131,072
 // triangles, 8 steps) and 5.6 GB 1.7 to 100 ms beside 25 (TE p = 3, 199,712
-// triangles, 32 steps), by the box.  So a handle's buffers stay for its next
-// solve, but only where they are in nobody's way:
+// triangles, 32 steps), by the box.  So a solve's buffers stay for the next
+// solve on the device, but only where they are in nobody's way:
 //   bounded     all idle buffers of a device together hold at most `limit`
 //               bytes; the oldest go first, and larger ones are never kept
 //   given back  with their handle or its mesh, on request, and whenever an
 //               allocation of the library fails on that device, whichever
 //               handle or ensemble makes it (reclaim, then the allocation again)
-//   safe        only idle buffers are here: a solve takes its handle's out and
-//               is their one owner until it gives them back.  Any thread may
-//               call; the memory itself is freed outside the lock.
+//   safe        only idle buffers are here, whose last solve has been waited
+//               for: a solve takes one out and is its one owner until it gives
+//               it back.  Any thread may call; the memory itself is freed
+//               outside the lock.
 // Host code without HIP: FREE is what frees a buffer.
 #pragma once
 
@@ -54,20 +55,28 @@ class KeptBuffers {
   }
 
  public:
-  // the owner's buffer, out of here (nullptr: none); *bytes its size
-  void *take(const void *owner, size_t *bytes) {
+  // a buffer of the device with room for `need`, out of here (nullptr: none);
+  // *bytes its size.  The owner's own, or the smallest of the others': handles
+  // that solve in turn share one.
+  void *take(const void *owner, int device, size_t need, size_t *bytes) {
     std::lock_guard<std::mutex> l(m);
-    for (size_t i = 0; i < v.size(); i++)
+    size_t best = v.size();
+    for (size_t i = 0; i < v.size(); i++) {
+      if (v[i].device != device || v[i].bytes < need) continue;
       if (v[i].owner == owner) {
-        void *p = v[i].p;
-        *bytes = v[i].bytes;
-        v.erase(v.begin() + (ptrdiff_t)i);
-        return p;
+        best = i;
+        break;
       }
+      if (best == v.size() || v[i].bytes < v[best].bytes) best = i;
+    }
     *bytes = 0;
-    return nullptr;
+    if (best == v.size()) return nullptr;
+    void *p = v[best].p;
+    *bytes = v[best].bytes;
+    v.erase(v.begin() + (ptrdiff_t)best);
+    return p;
   }
-  // an idle buffer of the owner's, its only one (std::bad_alloc: nothing done)
+  // a buffer that the owner is done with (std::bad_alloc: nothing done)
   void give(const void *owner, int device, void *p, size_t bytes, size_t limit) {
     if (bytes > limit) {
       FREE(p);

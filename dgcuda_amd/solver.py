@@ -280,8 +280,9 @@ class Solver:
         return J.value, gu, ge
 
     def adjoint_release(self):
-        """frees the device buffers that adjoint_solve has left for the next
-        solve (before another library's large allocation, for instance)"""
+        """frees the device buffers that this solver's last adjoint_solve has
+        left for the next one (before another library's large allocation, for
+        instance)"""
         self._chk(self.lib.dg_adjoint_release(self.h))
 
     def adjoint_rhs(self, u, gk, t=0.0, dt=1.0):

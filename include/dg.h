@@ -231,10 +231,11 @@ int dg_adjoint_set_objective(dg_handle *h, int kind, const double *params, int n
    at the final state. */
 int dg_adjoint_solve(dg_handle *h, int nsteps, double dt, int every, double *J,
                      double *grad_u0, double *grad_eps, int where);
-/* frees the work buffers that dg_adjoint_solve has left for the handle's next
-   solve.  All handles of a device together keep at most 1/32 of its memory;
-   kept buffers also go with the handle or its mesh, and when an allocation of
-   any handle or ensemble on the device fails (which is then made again).
+/* frees the work buffers that the handle's last dg_adjoint_solve has left for
+   the device's next one.  All handles of a device together leave at most 1/32
+   of its memory; the buffers also go with the handle or its mesh, and when an
+   allocation of any handle or ensemble on the device fails (which is then made
+   again).
    Allocations outside this library do not see them. */
 int dg_adjoint_release(dg_handle *h);
 /* one vector-Jacobian product of the right-hand side: gu = (dk/du)^T gk for

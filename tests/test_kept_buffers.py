@@ -26,7 +26,7 @@ static dgk::KeptBuffers<buf_free> K;
 int main() {
   int h[4];
   size_t n = 9;
-  CHECK(!K.take(&h[0], &n) && n == 0);
+  CHECK(!K.take(&h[0], 0, 1, &n) && n == 0);
   Buf *a = fresh(), *b = fresh(), *c = fresh(), *d = fresh();
   K.give(&h[0], 0, a, 40, 100);
   K.give(&h[1], 0, b, 50, 100);
@@ -34,17 +34,33 @@ int main() {
   CHECK(live == 4 && K.idle(0) == 90 && K.idle(1) == 100 && K.idle(2) == 0);
   K.give(&h[3], 0, d, 60, 100);           // 150: the oldest goes, then the next
   CHECK(a->state == 2 && b->state == 2 && c->state == 0 && live == 2);
-  CHECK(K.take(&h[0], &n) == nullptr && K.take(&h[3], &n) == d && n == 60);
+  CHECK(K.take(&h[3], 0, 61, &n) == nullptr && K.take(&h[3], 2, 1, &n) == nullptr);
+  CHECK(K.take(&h[3], 0, 60, &n) == d && n == 60);
   K.give(&h[3], 0, d, 101, 100);          // larger than the bound: not kept
-  CHECK(d->state == 2 && K.take(&h[3], &n) == nullptr && live == 1);
+  CHECK(d->state == 2 && K.take(&h[3], 0, 1, &n) == nullptr && live == 1);
   CHECK(K.idle(0) == 0 && !K.reclaim(0) && K.reclaim(1) && c->state == 2 && !K.reclaim(1) && live == 0);
   a = fresh(); b = fresh();
   K.give(&h[0], 0, a, 10, 100);
   K.give(&h[1], 0, b, 10, 100);
   K.drop(&h[0]);
-  CHECK(a->state == 2 && b->state == 0 && K.take(&h[1], &n) == b);
+  CHECK(a->state == 2 && b->state == 0 && K.take(&h[1], 0, 10, &n) == b);
   K.give(&h[1], 0, b, 10, 100);
   K.drop(&h[1]);
+  CHECK(live == 0);
+  // another handle's: its own first, else the smallest with room, now its own
+  a = fresh(); b = fresh(); c = fresh();
+  K.give(&h[0], 0, a, 30, 100);
+  K.give(&h[1], 0, b, 20, 100);
+  K.give(&h[2], 0, c, 10, 100);
+  CHECK(K.take(&h[0], 0, 5, &n) == a && n == 30);
+  CHECK(K.take(&h[3], 0, 11, &n) == b && n == 20);
+  K.give(&h[3], 0, b, 20, 100);
+  K.drop(&h[1]);
+  CHECK(b->state == 0);
+  K.drop(&h[3]);
+  CHECK(b->state == 2 && K.take(&h[3], 0, 10, &n) == c);
+  buf_free(a);
+  buf_free(c);
   CHECK(live == 0);
   // eight owners on two devices, each its own thread
   std::vector<std::thread> t;
@@ -58,8 +74,8 @@ int main() {
         if ((r >> 24) < 16) K.reclaim(dev);
         if ((r >> 24) > 250) K.drop(&own[i]);
         size_t have, need = 1 + (r >> 8) % 60;
-        Buf *p = (Buf *)K.take(&own[i], &have);
-        if (p && have < need) { buf_free(p); p = nullptr; }
+        Buf *p = (Buf *)K.take(&own[i], dev, need, &have);
+        if (p && have < need) { std::puts("too small"); std::abort(); }
         if (!p) { p = fresh(); have = need; }
         int idle = 0;
         if (!p->state.compare_exchange_strong(idle, 1)) { std::puts("two owners"); std::abort(); }
@@ -68,7 +84,8 @@ int main() {
       }
     });
   for (auto &x : t) x.join();
-  for (auto &o : own) K.drop(&o);
+  K.reclaim(0);
+  K.reclaim(1);
   CHECK(live == 0);
   std::puts("ok");
   return 0;
