@@ -3,7 +3,7 @@
 // A solve's work buffers are gigabytes that live for milliseconds: allocating
 // and freeing 1 GB took 1 to 28 ms beside 8 ms of gradient (Euler p = 4, 131,072
 // triangles, 8 steps) and 5.6 GB 1.7 to 100 ms beside 25 (TE p = 3, 199,712
-// triangles, 32 steps), by the box.  So a solve's buffers stay for the next
+// triangles, 32 steps), by the machine.  So a solve's buffers stay for the next
 // solve on the device, but only where they are in nobody's way:
 //   bounded     all idle buffers of a device together hold at most `limit`
 //               bytes; the oldest go first, and larger ones are never kept
